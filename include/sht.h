@@ -223,6 +223,41 @@ int sht_batch_launch(sht_batch *batch, void *stream);
 int sht_batch_uses_graph(const sht_batch *batch);
 int sht_batch_destroy(sht_batch *batch);
 
+/* The dry primitive-equation core around its transforms (dycore.py; no single reference call:
+ * the tendency pipeline of SpeedyWeather/src/dynamics/tendencies.jl:119-177 and the leapfrog of
+ * time_stepping/steppers/leapfrog.jl:175-286 without physics), E members of L equally spaced
+ * sigma levels.  Prognostic columns: vorticity, divergence, temperature (E L columns each,
+ * member by member) and ln ps (E), each column nharm complex floats one after another; all
+ * pointers but the descriptor's own are device pointers. */
+typedef struct sht_dry_model {
+    int32_t nlayers;            /* L */
+    int32_t nmembers;           /* E */
+    double radius;              /* m */
+    double r_dry;               /* gas constant */
+    double kappa;               /* r_dry / cp */
+    const float *coslat_inv;    /* 1 / cos(lat) of every grid point */
+    const float *coriolis;      /* Coriolis parameter of every grid point */
+    const float *geopotential;  /* L x L, row-major: Phi_k = sum over j >= k of G[k][j] T_j */
+} sht_dry_model;
+/* Spectral tendencies of a state into tend (3 E L + E columns: vorticity, divergence,
+ * temperature, ln ps).  The caller's workspaces: spec, at least max(5 E L + 3 E, 6 E L + E)
+ * spectral columns; grid, 5 E L + 2 E grid columns (3 E with with_grid); fields, 6 E L + E
+ * grid columns.  With with_grid, grid holds on return u, v (E L columns each), then 2 E
+ * columns of the ln ps gradient, T, divergence, vorticity (E L each) and ln ps (E).
+ * The plan's nlayers must cover those column counts.  Asynchronous on `stream`. */
+int sht_dry_tendencies(sht_plan *plan, const sht_dry_model *model, const void *vor, const void *div, const void *temp,
+                       const void *lnps, void *tend, void *spec, void *grid, void *fields, int32_t with_grid,
+                       void *stream);
+/* One time step of the columns (as four arrays: vorticity, divergence, temperature, ln ps):
+ * next = (base + dt2 tend) / (1 + dt2 nu) with base = prev[] if not null, else state[];
+ * nu_div damps the divergence, nu vorticity and temperature, ln ps is not damped.  With
+ * prev: d = prev - 2 state + next, filtered = state + w1 d, next -= w2 d (Robert-Asselin-
+ * Williams).  filtered (only written with prev) and next: 3 E L + E columns, not aliasing
+ * any input. */
+int sht_dry_leapfrog(sht_plan *plan, int32_t nlayers, int32_t nmembers, const void *const *state,
+                     const void *const *prev, const void *tend, const float *nu, const float *nu_div, double dt2,
+                     double w1, double w2, void *filtered, void *next, void *stream);
+
 /* Learned column correction (an addition of this library; no reference counterpart): an MLP
  * 32 -> 128 -> 128 -> 32 with GELU per grid column (8 levels x {u, v, T, ln ps}), BF16
  * weights with FP32 master copy and FP32 accumulation, trained with Adam on the mean

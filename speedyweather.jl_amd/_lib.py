@@ -31,6 +31,7 @@ EXPORTS = (
     "sht_grid2spec_pullback", "sht_divergence", "sht_laplace", "sht_gradient", "sht_plan_create_matrix",
     "sht_synthesis_laplace", "sht_analysis_laplace", "sht_time_stage", "sht_tune_cache_save",
     "sht_tune_cache_load", "sht_transform_static", "sht_plan_set_graphs", "sht_plan_graph_count",
+    "sht_dry_tendencies", "sht_dry_leapfrog",
 )
 
 
@@ -63,6 +64,12 @@ SHT_BATCH_NO_GRAPH, SHT_BATCH_FORCE_GRAPH_FAILURE = 1, 2
 class ShtSizes(C.Structure):
     _fields_ = [("npoints", C.c_int64), ("nharm", C.c_int64), ("nlat", C.c_int32),
                 ("nlon_max", C.c_int32), ("nfreq_total", C.c_int64), ("device_bytes", C.c_int64)]
+
+
+class ShtDryModel(C.Structure):
+    _fields_ = [("nlayers", C.c_int32), ("nmembers", C.c_int32), ("radius", C.c_double), ("r_dry", C.c_double),
+                ("kappa", C.c_double), ("coslat_inv", C.c_void_p), ("coriolis", C.c_void_p),
+                ("geopotential", C.c_void_p)]
 
 
 _LIB = None
@@ -99,6 +106,8 @@ def lib() -> C.CDLL:
         L.sht_batch_launch.argtypes = [vp, vp]
         L.sht_batch_uses_graph.argtypes = [vp]
         L.sht_batch_destroy.argtypes = [vp]
+        L.sht_dry_tendencies.argtypes = [vp, C.POINTER(ShtDryModel)] + [vp] * 8 + [i32, vp]
+        L.sht_dry_leapfrog.argtypes = [vp, i32, i32] + [vp] * 5 + [C.c_double] * 3 + [vp] * 3
         L.sht_mlp_create.argtypes = [i32, i32, C.POINTER(vp)]
         L.sht_mlp_set_params.argtypes = [vp, vp]
         L.sht_mlp_get_params.argtypes = [vp, vp]

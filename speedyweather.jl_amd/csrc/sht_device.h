@@ -114,6 +114,39 @@ struct FastDiv {
     __device__ int div(int x) const { return d == 1 ? x : (int)__umulhi((unsigned)x, mul); }
 };
 
+// U, V = (u, v) cos(lat) of packed coefficient lm on the unit sphere from the column's
+// vorticity and divergence (spectral_gradients.jl:331-366): a 3-point stencil in l.
+__device__ __forceinline__ void uv_stencil(const DevPlan &P, const SHT_GLOBAL float2 *vor, const SHT_GLOBAL float2 *dv,
+                                           int lm, float2 &uu, float2 &vv) {
+    const int l = as_global(P.l_of)[lm];
+    const float x = as_global(P.uv_x)[lm], u1 = as_global(P.uv_1)[lm], u2 = as_global(P.uv_2)[lm];
+    const float2 z = gload(vor + lm), d = gload(dv + lm);
+    float2 du = make_float2(0.f, 0.f), dvv = make_float2(0.f, 0.f);
+    // i x D and i x ζ
+    if (lm == 0) {
+        float2 zp = make_float2(0.f, 0.f), dp = make_float2(0.f, 0.f);
+        if (P.lmax > 1) {
+            zp = gload(vor + 1);
+            dp = gload(dv + 1);
+        }
+        uu = make_float2(-x * d.y + u2 * zp.x, x * d.x + u2 * zp.y);
+        vv = make_float2(-x * z.y - u2 * dp.x, x * z.x - u2 * dp.y);
+    } else if (l == P.lmax - 1) {
+        const float2 zm = gload(vor + lm - 1), dm = gload(dv + lm - 1);
+        uu = make_float2(-u1 * zm.x, -u1 * zm.y);
+        vv = make_float2(u1 * dm.x, u1 * dm.y);
+    } else {
+        const float2 zm = gload(vor + lm - 1), dm = gload(dv + lm - 1);
+        if (l < P.lmax - 2) {
+            du = gload(vor + lm + 1);
+            dvv = gload(dv + lm + 1);
+        }
+        // u2 is 0 on the second-to-last row, so du, dvv only enter below it
+        uu = make_float2(-x * d.y + u2 * du.x - u1 * zm.x, x * d.x + u2 * du.y - u1 * zm.y);
+        vv = make_float2(-x * z.y + u1 * dm.x - u2 * dvv.x, x * z.x + u1 * dm.y - u2 * dvv.y);
+    }
+}
+
 static inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 }  // namespace sht

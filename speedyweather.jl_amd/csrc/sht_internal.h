@@ -98,7 +98,7 @@ constexpr int kXCDs = 8;
 struct CallArgs {
     int plan;             // index into the launch's plan array
     int K;                // columns
-    int unscale;          // synthesis: divide by cos(lat)
+    int unscale;          // synthesis: divide by cos(lat); mixed: the leading columns that are
     int paired;           // single-call FFT synthesis: a ring's column groups on one XCD
     const void *in;       // synthesis: coefficients; analysis: grid
     void *out;            // synthesis: grid; analysis: coefficients
@@ -119,6 +119,7 @@ struct CallArgs {
     int lap;
     float lap_sign;
     float lap_scale;
+    int mixed;            // single-call synthesis: only the first `unscale` columns are unscaled
 };
 
 enum Stage { kLegendreSynthesis = 0, kFFTSynthesis = 1, kFFTAnalysis = 2, kLegendreAnalysis = 3 };
@@ -292,6 +293,7 @@ int static_scratch_setup(int device);
 // kernels read their tile from tiles[blockIdx.x], the FFT kernels derive ring and column
 // group from blockIdx.x.  batch = true: tile, call and column group from tiles.
 const void *legendre_kernel(int stage, int mode, bool batch);
+const void *legendre_mixed_kernel(int mode);  // single-call synthesis with CallArgs::mixed
 // accumulate: the single-call synthesis that adds into its output (pullbacks); batches
 // never accumulate.
 const void *fft_kernel(int stage, bool batch, bool accumulate = false);

@@ -226,7 +226,9 @@ __device__ inline unsigned char *ep_slot(unsigned char *sm, int rb) {
 
 // Four workgroups per CU: at most 128 registers per lane, and the per-ring epilogue factors
 // sit in the staging rows' padding, so LDS stays at 40 KiB (36 KiB in FP32).
-template <int MODE, bool BATCH>
+// MIXED: C.unscale leading columns are divided by cos(lat), the others not (its own
+// instantiation, so that the other calls keep one factor per ring).
+template <int MODE, bool BATCH, bool MIXED = false>
 __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthesis_kernel(const DevPlan *__restrict__ plans, CallArgs single,
                                                                  const CallArgs *__restrict__ calls,
                                                                  const Tile *__restrict__ tiles) {
@@ -367,6 +369,7 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
         unsigned char *slot = ep_slot<MODE>(sm, lane);
         *reinterpret_cast<long long *>(slot) = e_row;
         *reinterpret_cast<float *>(slot + 8) = e_sc * e_ci;
+        if constexpr (MIXED) *reinterpret_cast<float *>(slot + 12) = e_sc;
     }
     int c = 0;
     for (; c + 1 < nch; c += 2) {
@@ -398,7 +401,7 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
             const int j = j0 + 16 * tile + r;
             const int rb = 16 * w + r;  // ring within the block
             const unsigned char *slot = ep_slot<MODE>(sm, rb);
-            const float sc = *reinterpret_cast<const float *>(slot + 8);
+            const float sc = *reinterpret_cast<const float *>(slot + (MIXED && k >= unscale ? 12 : 8));
             const float e = acc[0][cb][i] * sc, o = acc[1][cb][i] * sc;
             const float nv = e + o, sv = e - o;
             const float n_other = lane_xor1(nv);
@@ -652,6 +655,12 @@ static const void *legendre_entry(int stage, bool batch) {
                      : reinterpret_cast<const void *>(&legendre_synthesis_kernel<MODE, false>);
     return batch ? reinterpret_cast<const void *>(&legendre_analysis_kernel<MODE, true>)
                  : reinterpret_cast<const void *>(&legendre_analysis_kernel<MODE, false>);
+}
+
+const void *legendre_mixed_kernel(int mode) {
+    if (mode == kFP32) return reinterpret_cast<const void *>(&legendre_synthesis_kernel<kFP32, false, true>);
+    if (mode == kFP16x3) return reinterpret_cast<const void *>(&legendre_synthesis_kernel<kFP16x3, false, true>);
+    return reinterpret_cast<const void *>(&legendre_synthesis_kernel<kBF16x3, false, true>);
 }
 
 const void *legendre_kernel(int stage, int mode, bool batch) {

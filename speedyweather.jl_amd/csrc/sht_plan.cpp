@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/sht.h"
+#include "sht_dycore.h"
 #include "sht_internal.h"
 
 using sht::CallArgs;
@@ -1269,7 +1270,9 @@ static StageLaunch plan_stage_launch(const sht_plan *plan, int stage, const Call
     const int gx = plan->leg_xcd;
     switch (stage) {
         case sht::kLegendreSynthesis:
-            return {sht::legendre_kernel(stage, plan->d.precision, false), dim3(plan->nsyn[gx][cgs - 1]), 0,
+            return {c.mixed ? sht::legendre_mixed_kernel(plan->d.precision)
+                            : sht::legendre_kernel(stage, plan->d.precision, false),
+                    dim3(plan->nsyn[gx][cgs - 1]), 0,
                     plan->syn_tiles[gx][cgs - 1]};
         case sht::kFFTSynthesis:
         case sht::kFFTAnalysis: {
@@ -1320,7 +1323,7 @@ static bool launch_from_graph(sht_plan *plan, int dir, int s0, int s1, const Cal
     std::string key;
     auto put = [&key](const auto &v) { key.append(reinterpret_cast<const char *>(&v), sizeof(v)); };
     put(c.K), put(c.unscale), put(c.paired), put(c.in), put(c.out), put(c.ld_in), put(c.ld_out), put(c.fbuf);
-    put(c.adj), put(c.accumulate), put(c.lap), put(c.lap_sign), put(c.lap_scale);
+    put(c.adj), put(c.accumulate), put(c.lap), put(c.lap_sign), put(c.lap_scale), put(c.mixed);
     put(plan->pol), put(plan->leg_xcd), put(plan->fft_pair), put(plan->fourier), put(plan->dft_cg);
     hipGraphExec_t exec = nullptr;
     {
@@ -1379,10 +1382,11 @@ static void *call_scratch(sht_plan *plan, void *scratch, void *stream) {
 
 // Spectral -> grid stages (Legendre synthesis, FFT synthesis); adj = 2 and accumulate turn
 // them into the pullback of the analysis; op fuses a Laplacian of the input; scratch (if
-// not null) replaces the stream's scratch.
+// not null) replaces the stream's scratch; unscale_cols > 0 divides only that many leading
+// columns by cos(lat) (on the regular kernels, also on a matrix plan).
 static int run_synthesis(sht_plan *plan, const void *coeffs, int64_t ld_spec, void *field, int64_t ld_grid, int32_t K,
                          int32_t unscale_coslat, int adj, int accumulate, void *stream, LapOp op = LapOp(),
-                         void *scratch = nullptr) {
+                         void *scratch = nullptr, int unscale_cols = 0) {
     int rc = check_call(plan, coeffs, field, K);
     if (rc) return rc;
     if (ld_spec < plan->g.nharm) return fail(SHT_ERR_DIM, "DimensionMismatch: ld_spec < nharm");
@@ -1390,7 +1394,7 @@ static int run_synthesis(sht_plan *plan, const void *coeffs, int64_t ld_spec, vo
     DeviceGuard guard(plan->d.device);
     void *ws = call_scratch(plan, scratch, stream);
     if (!ws) return SHT_ERR_ALLOC;
-    if (plan->matrix && adj == 0 && !accumulate && op.lap == 0) {  // field = B_int a_int, one GEMM (rows / cos(lat))
+    if (plan->matrix && adj == 0 && !accumulate && op.lap == 0 && unscale_cols == 0) {  // field = B_int a_int, one GEMM (rows / cos(lat))
         float *work = static_cast<float *>(ws);  // the GEMM needs no Fourier buffer
         rc = sht::launch_dense_gemm(plan->mat_syn, plan->g.npoints, 2 * plan->g.nharm,
                                     static_cast<const float *>(coeffs), 2 * ld_spec, K, static_cast<float *>(field),
@@ -1398,8 +1402,8 @@ static int run_synthesis(sht_plan *plan, const void *coeffs, int64_t ld_spec, vo
         if (rc) return fail(SHT_ERR_HIP, std::string("dense synthesis launch: ") + hipGetErrorString((hipError_t)rc));
         return SHT_OK;
     }
-    const CallArgs c{0, K, unscale_coslat ? 1 : 0, plan->fft_pair, coeffs, field, ld_spec, ld_grid, ws,
-                     adj, accumulate ? 1 : 0, op.lap, op.sign, op.scale};
+    const CallArgs c{0, K, unscale_cols > 0 ? unscale_cols : (unscale_coslat ? 1 : 0), plan->fft_pair, coeffs, field,
+                     ld_spec, ld_grid, ws, adj, accumulate ? 1 : 0, op.lap, op.sign, op.scale, unscale_cols > 0 ? 1 : 0};
     hipError_t e;
     if (launch_from_graph(plan, 0, sht::kLegendreSynthesis, sht::kFFTSynthesis, c, stream, e)) {
         if (e != hipSuccess) return fail(SHT_ERR_HIP, std::string("synthesis graph launch: ") + hipGetErrorString(e));
@@ -1433,7 +1437,7 @@ static int run_analysis(sht_plan *plan, const void *field, int64_t ld_grid, void
         return SHT_OK;
     }
     const CallArgs c{0,  K,   unscale_coslat ? 1 : 0, 0,      field,   coeffs, ld_grid, ld_spec,
-                     ws, adj, accumulate ? 1 : 0,     op.lap, op.sign, op.scale};
+                     ws, adj, accumulate ? 1 : 0,     op.lap, op.sign, op.scale, 0};
     hipError_t e;
     if (launch_from_graph(plan, 1, sht::kFFTAnalysis, sht::kLegendreAnalysis, c, stream, e)) {
         if (e != hipSuccess) return fail(SHT_ERR_HIP, std::string("analysis graph launch: ") + hipGetErrorString(e));
@@ -1579,6 +1583,71 @@ int sht_gradient(sht_plan *plan, const void *p, void *dpdx, void *dpdy, int64_t 
     rc = sht::launch_spectral_op(plan->dP, plan->g.nharm, sht::kOpGradient, p, nullptr, dpdx, dpdy, ld, K, 0,
                                  (float)(1.0 / radius), stream);
     if (rc) return fail(SHT_ERR_HIP, std::string("gradient launch: ") + hipGetErrorString((hipError_t)rc));
+    return SHT_OK;
+}
+
+static int check_dry(sht_plan *plan, int32_t L, int32_t E) {
+    if (!plan) return fail(SHT_ERR_ARG, "null plan");
+    if (L < 1 || E < 1 || (long long)E * (6 * (long long)L + 2) > 0x7fffffffLL)
+        return fail(SHT_ERR_DIM, "DimensionMismatch: " + std::to_string(L) + " levels of " + std::to_string(E) + " members");
+    return SHT_OK;
+}
+
+int sht_dry_tendencies(sht_plan *plan, const sht_dry_model *model, const void *vor, const void *div, const void *temp,
+                       const void *lnps, void *tend, void *spec, void *grid, void *fields, int32_t with_grid,
+                       void *stream) {
+    sht::TraceRange trace_range("sht_dry_tendencies");
+    if (!model) return fail(SHT_ERR_ARG, "null model");
+    const int L = model->nlayers, E = model->nmembers;
+    int rc = check_dry(plan, L, E);
+    if (rc) return rc;
+    if (!vor || !div || !temp || !lnps || !tend || !spec || !grid || !fields || !model->coslat_inv ||
+        !model->coriolis || !model->geopotential)
+        return fail(SHT_ERR_ARG, "null data pointer");
+    if (!(model->radius > 0)) return fail(SHT_ERR_ARG, "radius must be positive");
+    const int nharm = plan->g.nharm, np = (int)plan->g.npoints;
+    const int down = 5 * E * L + (with_grid ? 3 : 2) * E, up = 6 * E * L + E;
+    const sht::DryState st{static_cast<const float2 *>(vor), static_cast<const float2 *>(div),
+                           static_cast<const float2 *>(temp), static_cast<const float2 *>(lnps)};
+    DeviceGuard guard(plan->d.device);
+    if ((rc = check_call(plan, spec, grid, std::max(down, up)))) return rc;
+    auto launched = [](int e, const char *what) {
+        return e ? fail(SHT_ERR_HIP, std::string(what) + " launch: " + hipGetErrorString((hipError_t)e)) : SHT_OK;
+    };
+    rc = launched(sht::launch_dry_columns(plan->dP, nharm, st, spec, L, E, (float)model->radius, stream), "dry columns");
+    if (rc) return rc;
+    // u, v and the ln ps gradient carry cos(lat), the other columns do not
+    rc = run_synthesis(plan, spec, nharm, grid, np, down, 0, 0, 0, stream, LapOp(), nullptr, 2 * E * L + 2 * E);
+    if (rc) return rc;
+    rc = launched(sht::launch_dry_grid(static_cast<const float *>(grid), static_cast<float *>(fields), model->coslat_inv,
+                                       model->coriolis, np, L, E, 1.f / (float)model->radius, (float)model->r_dry,
+                                       (float)model->kappa, stream),
+                  "dry grid tendencies");
+    if (rc) return rc;
+    if ((rc = run_analysis(plan, fields, np, spec, nharm, up, 0, 0, 0, stream))) return rc;
+    return launched(sht::launch_dry_tendency(plan->dP, nharm, spec, st.temp, model->geopotential, tend, L, E,
+                                             model->radius, stream),
+                    "dry spectral tendencies");
+}
+
+int sht_dry_leapfrog(sht_plan *plan, int32_t nlayers, int32_t nmembers, const void *const *state,
+                     const void *const *prev, const void *tend, const float *nu, const float *nu_div, double dt2,
+                     double w1, double w2, void *filtered, void *next, void *stream) {
+    sht::TraceRange trace_range("sht_dry_leapfrog");
+    int rc = check_dry(plan, nlayers, nmembers);
+    if (rc) return rc;
+    if (!state || !tend || !nu || !nu_div || !next || (prev && !filtered)) return fail(SHT_ERR_ARG, "null data pointer");
+    for (int i = 0; i < 4; ++i)
+        if (!state[i] || (prev && !prev[i])) return fail(SHT_ERR_ARG, "null data pointer");
+    auto columns = [](const void *const *p) {
+        return sht::DryState{static_cast<const float2 *>(p[0]), static_cast<const float2 *>(p[1]),
+                             static_cast<const float2 *>(p[2]), static_cast<const float2 *>(p[3])};
+    };
+    DeviceGuard guard(plan->d.device);
+    rc = sht::launch_dry_leapfrog(plan->g.nharm, columns(state), columns(prev ? prev : state), tend, nu, nu_div,
+                                  filtered, next, nlayers, nmembers, (float)dt2, (float)w1, (float)w2, prev ? 1 : 0,
+                                  stream);
+    if (rc) return fail(SHT_ERR_HIP, std::string("dry leapfrog launch: ") + hipGetErrorString((hipError_t)rc));
     return SHT_OK;
 }
 

@@ -27,7 +27,9 @@ a correspondingly shorter time step.
 Spectral operators follow SpeedyTransforms/src/spectral_gradients.jl:30-125 (curl and
 divergence of a vector whose grid components carry a 1/cos(lat) factor), :386-421
 (Laplacian) and :483-527 (gradient), with the factors of gradient_arrays.jl:4-145.
-Every spectral <-> grid transform runs on the engine; grid-point arithmetic uses torch.
+Every spectral <-> grid transform runs on the engine, and so do the tendencies and the time
+step (sht_dry_tendencies, sht_dry_leapfrog: one kernel per pass over the data between the
+transforms); setup and initial states use torch.
 """
 from __future__ import annotations
 
@@ -37,7 +39,7 @@ import math
 import numpy as np
 import torch
 
-from ._lib import lib
+from ._lib import DimensionMismatch, ShtDryModel, check, lib
 from .grids import OctahedralGaussianGrid, get_nlat_half
 from .spectrum import LowerTriangularArray, Spectrum
 from .transform import SpectralTransform, UV_from_vordiv_, transform_
@@ -129,7 +131,8 @@ class DryPrimitiveModel:
         self.grid = OctahedralGaussianGrid(get_nlat_half(trunc + 1))
         self.a = radius
         L, E = nlayers, nmembers
-        self.S = SpectralTransform(self.spectrum, self.grid, nlayers=E * (6 * L + 1), precision=precision,
+        # columns of a tendency's transforms: 5 L + 3 fields to the grid, 6 L + 1 back
+        self.S = SpectralTransform(self.spectrum, self.grid, nlayers=E * max(6 * L + 1, 5 * L + 3), precision=precision,
                                    device=self.device.index or 0)
         self.ops = SpectralOps(self.spectrum, self.device)
         lat = grid_latitudes(self.grid)
@@ -188,66 +191,57 @@ class DryPrimitiveModel:
         return U, V
 
     # ------------------------------------------------------------------ dynamics
+    def _columns(self, st: dict, what: str):
+        """Device pointers of a state's vor, div, temp (E*L, nharm) and lnps (E, nharm), and the
+        tensors that hold them."""
+        E, EL, n = self.E, self.E * self.L, self.spectrum.nharm
+        keep, ptr = [], []
+        for name, rows in (("vor", EL), ("div", EL), ("temp", EL), ("lnps", E)):
+            t = st[name]
+            if t.dtype != torch.complex64:
+                raise TypeError(f"{what} {name} has dtype {t.dtype}, the model needs {torch.complex64}")
+            if tuple(t.shape) != (rows, n):
+                raise DimensionMismatch(f"{what} {name} is {tuple(t.shape)}, the model needs {(rows, n)}")
+            if t.device != self.coslat.device:
+                raise ValueError(f"{what} {name} is on {t.device}, the model on {self.coslat.device}")
+            t = t.resolve_conj().contiguous()
+            keep.append(t)
+            ptr.append(t.data_ptr())
+        return ptr, keep
+
+    def _split(self, x: torch.Tensor) -> dict:
+        """The columns vor, div, temp (E*L each) and lnps (E) of one tensor."""
+        EL = self.E * self.L
+        vor, div, temp, lnps = x.split((EL, EL, EL, self.E))
+        return {"vor": vor, "div": div, "temp": temp, "lnps": lnps}
+
+    def _vector(self, x: torch.Tensor) -> torch.Tensor:
+        return x.to(device=self.coslat.device, dtype=torch.float32).contiguous()
+
     def tendencies(self, st: dict, with_grid: bool = False):
-        """Spectral tendencies of vor, div, temp (E*L, nharm) and lnps (E, nharm)."""
-        L, E, a = self.L, self.E, self.a
-        ops = self.ops
-        vor, div, temp, lnps = st["vor"], st["div"], st["temp"], st["lnps"]
-        U, V = self.uv(vor, div)
-        g1 = self.synth(torch.cat([U, V, ops.dlambda(lnps), ops.coslat_dlat(lnps)]), unscale=True)
-        g2 = self.synth(torch.cat([temp, div, vor, lnps]))
-        EL = E * L
-        u, v = g1[:EL].view(E, L, -1), g1[EL:2 * EL].view(E, L, -1)
-        dqdx, dqdy = (g1[2 * EL:2 * EL + E] / a).view(E, 1, -1), (g1[2 * EL + E:] / a).view(E, 1, -1)
-        T, D, Z = g2[:EL].view(E, L, -1), g2[EL:2 * EL].view(E, L, -1), g2[2 * EL:3 * EL].view(E, L, -1)
-        q = g2[3 * EL:].view(E, 1, -1)
-        ds = self.dsigma
-        uq = u * dqdx + v * dqdy                      # (u, v) . grad ln ps
-        dsum = ds * (D + uq)                          # layer mass-flux divergence
-        csum = torch.cumsum(dsum, dim=1)
-        lnps_t = -csum[:, -1:, :]                     # d ln ps / dt
-        sh = self.sigma_half.view(1, -1, 1)
-        sdot = torch.zeros((E, L + 1, u.shape[-1]), device=self.device)
-        sdot[:, 1:L] = -csum[:, :L - 1] - sh[:, 1:L] * lnps_t
-        def vadv(X):
-            dX = X[:, 1:] - X[:, :-1]                 # (E, L-1)
-            out = torch.zeros_like(X)
-            out[:, :-1] += sdot[:, 1:L] * dX
-            out[:, 1:] += sdot[:, 1:L] * dX
-            return out / (2 * ds)
-        sf = self.sigma_full.view(1, -1, 1)
-        omp = uq - (csum - 0.5 * dsum) / sf           # omega / p on full levels
-        absvor = Z + self.f
-        Au = absvor * v - vadv(u) - R_DRY * T * dqdx
-        Av = -absvor * u - vadv(v) - R_DRY * T * dqdy
-        ke = 0.5 * (u * u + v * v)
-        Tt = T * D - vadv(T) + KAPPA * T * omp
-        ci = self.coslat_inv
-        flds = torch.cat([(Au * ci).view(EL, -1), (Av * ci).view(EL, -1), (u * T * ci).view(EL, -1),
-                          (v * T * ci).view(EL, -1), ke.view(EL, -1), Tt.view(EL, -1), lnps_t.view(E, -1)])
-        s = self.analyse(flds)
-        Aus, Avs, uTs, vTs, kes, Tts = (s[i * EL:(i + 1) * EL] for i in range(6))
-        lnps_ts = s[6 * EL:].clone()
-        phi = torch.einsum("kj,ejn->ekn", self.G.to(torch.complex64),
-                           temp.view(E, L, -1)).reshape(EL, -1)
-        vor_t = ops.curl(Aus, Avs) / a
-        div_t = ops.divergence(Aus, Avs) / a - ops.laplace(phi + kes) / (a * a)
-        temp_t = -ops.divergence(uTs, vTs) / a + Tts
-        lnps_ts[:, 0] = 0                              # global mass conservation
-        # the extra degree only serves the vector path: no prognostic tendency there
-        keep = ops.keep
-        tend = {"vor": vor_t * keep, "div": div_t * keep, "temp": temp_t * keep, "lnps": lnps_ts * keep}
+        """Spectral tendencies of vor, div, temp (E*L, nharm) and lnps (E, nharm); with_grid
+        also u, v, T (E, L, npoints) and lnps (E, 1, npoints)."""
+        L, E = self.L, self.E
+        EL, n, npts, dev = E * L, self.spectrum.nharm, self.grid.npoints, self.coslat.device
+        ptr, keep = self._columns(st, "state")
+        tables = [self._vector(t) for t in (self.coslat_inv, self.f, self.G)]
+        model = ShtDryModel(L, E, self.a, R_DRY, KAPPA, *(t.data_ptr() for t in tables))
+        down, up = 5 * EL + (3 if with_grid else 2) * E, 6 * EL + E
+        tend = torch.empty((3 * EL + E, n), dtype=torch.complex64, device=dev)
+        spec = torch.empty((max(5 * EL + 3 * E, up), n), dtype=torch.complex64, device=dev)
+        g = torch.empty((down, npts), device=dev)
+        fields = torch.empty((up, npts), device=dev)
+        check(lib().sht_dry_tendencies(self.S._plan, C.byref(model), *ptr, tend.data_ptr(), spec.data_ptr(),
+                                       g.data_ptr(), fields.data_ptr(), int(bool(with_grid)), self.S._stream()),
+              "sht_dry_tendencies")
+        out = self._split(tend)
         if with_grid:
-            return tend, {"u": u, "v": v, "T": T, "lnps": q}
-        return tend
+            o = 2 * EL + 2 * E
+            return out, {"u": g[:EL].view(E, L, -1), "v": g[EL:2 * EL].view(E, L, -1),
+                         "T": g[o:o + EL].view(E, L, -1), "lnps": g[o + 3 * EL:].view(E, 1, -1)}
+        return out
 
     # ------------------------------------------------------------------ time stepping
-    def _diffuse(self, name, x, dt2):
-        nu = self.nu_div if name == "div" else self.nu
-        if name == "lnps":
-            return x
-        return x / (1.0 + dt2 * nu)
-
     def step(self, correction=None):
         """One leapfrog step (Euler forward for the first); `correction(model, tend, grid)`
         may add to the spectral tendencies."""
@@ -256,19 +250,29 @@ class DryPrimitiveModel:
         tend, grid = (out if need_grid else (out, None))
         if correction is not None:
             correction(self, tend, grid)
+        L, E, n, dev = self.L, self.E, self.spectrum.nharm, self.coslat.device
+        rows = 3 * E * L + E
+        tptr, tkeep = self._columns(tend, "tendency")
+        if any(p != tptr[0] + 8 * n * E * L * i for i, p in enumerate(tptr)):  # a correction put its own tensors there
+            tkeep = torch.cat(tkeep)
+            tptr = [tkeep.data_ptr()]
+        sptr, skeep = self._columns(self.state, "state")
+        nu, nu_div = self._vector(self.nu), self._vector(self.nu_div)
+        arr = C.c_void_p * 4
+        new = torch.empty((rows, n), dtype=torch.complex64, device=dev)
         if self.state_prev is None:
-            dt2, base = self.dt, self.state
+            dt2, prev, filtered = self.dt, None, None
         else:
-            dt2, base = 2.0 * self.dt, self.state_prev
-        new = {k: self._diffuse(k, base[k] + dt2 * tend[k], dt2) for k in self.state}
-        if self.state_prev is not None:
-            w1 = self.robert * self.williams / 2
-            w2 = self.robert * (1 - self.williams) / 2
-            for k in self.state:
-                d = self.state_prev[k] - 2 * self.state[k] + new[k]
-                self.state[k] = self.state[k] + w1 * d
-                new[k] = new[k] - w2 * d
-        self.state_prev, self.state = self.state, new
+            pptr, pkeep = self._columns(self.state_prev, "previous state")
+            filtered = torch.empty_like(new)
+            dt2, prev = 2.0 * self.dt, arr(*pptr)
+        w1 = self.robert * self.williams / 2
+        w2 = self.robert * (1 - self.williams) / 2
+        check(lib().sht_dry_leapfrog(self.S._plan, L, E, arr(*sptr), prev, tptr[0], nu.data_ptr(), nu_div.data_ptr(),
+                                     dt2, w1, w2, None if filtered is None else filtered.data_ptr(), new.data_ptr(),
+                                     self.S._stream()), "sht_dry_leapfrog")
+        self.state_prev = self.state if filtered is None else self._split(filtered)
+        self.state = self._split(new)
         self.nsteps += 1
 
     # ------------------------------------------------------------------ initial conditions
