@@ -41,6 +41,8 @@ class _RingGrid:
         if nlat_half < 1:
             raise ValueError("nlat_half must be >= 1")
         self.nlat_half = int(nlat_half)
+        # every transform call compares sizes with it
+        self.npoints = 2 * sum(self.nlon_ring(j) for j in range(self.nlat_half))
 
     def nlon_ring(self, j: int) -> int:  # 0-based northern ring
         raise NotImplementedError
@@ -53,10 +55,6 @@ class _RingGrid:
     def nlons(self) -> np.ndarray:
         north = [self.nlon_ring(j) for j in range(self.nlat_half)]
         return np.array(north + north[::-1])
-
-    @property
-    def npoints(self) -> int:
-        return int(self.nlons.sum())
 
     @property
     def nlon_max(self) -> int:

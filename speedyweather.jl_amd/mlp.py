@@ -21,7 +21,7 @@ def nparams() -> int:
 
 
 def _stream(device):
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(device.index))
 
 
 def _check_rows(x: torch.Tensor, name: str, device) -> None:

@@ -129,26 +129,27 @@ class SpectralTransform:
 
     # -------------------------------------------------------------- checks
     def _stream(self):
-        return C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
+        # the current stream's handle without building a Stream object
+        return C.c_void_p(torch._C._cuda_getCurrentRawStream(self.device))
 
     def _check_tensor(self, t: torch.Tensor, n: int, dtype, what: str):
-        if not t.is_cuda or t.device.index != self.device:
+        if t.get_device() != self.device:  # -1: not on a GPU
             raise ValueError(f"{what} must be on cuda:{self.device} (the MI355X engine has no CPU path)")
         if t.dtype != dtype:
             raise TypeError(f"{what} has dtype {t.dtype}, transform needs {dtype}")
         t2 = t if t.dim() == 2 else t.unsqueeze(0)
-        if t2.stride(-1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < n):
-            raise ValueError(f"{what} must be contiguous along its last dimension")
         K = t2.shape[0]
-        ld = t2.stride(0) if K > 1 else n
-        return t2, K, ld
+        stride = t2.stride()
+        if stride[-1] != 1 or (K > 1 and stride[0] < n):
+            raise ValueError(f"{what} must be contiguous along its last dimension")
+        return t2, K, stride[0] if K > 1 else n
 
     def ismatching(self, x) -> bool:
         """Architectures.ismatching (spectral_transform.jl:387-403)."""
         if isinstance(x, LowerTriangularArray):
-            return x.spectrum == self.spectrum and x.nlayers <= self.nlayers
+            return (x.spectrum is self.spectrum or x.spectrum == self.spectrum) and x.nlayers <= self.nlayers
         if isinstance(x, Field):
-            return x.grid == self.grid and x.nlayers <= self.nlayers
+            return (x.grid is self.grid or x.grid == self.grid) and x.nlayers <= self.nlayers
         return False
 
 
@@ -437,7 +438,7 @@ class SpectralBatch:
         return bool(lib().sht_batch_uses_graph(self._batch))
 
     def launch(self):
-        check(lib().sht_batch_launch(self._batch, C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)),
+        check(lib().sht_batch_launch(self._batch, C.c_void_p(torch._C._cuda_getCurrentRawStream(self.device))),
               "sht_batch_launch")
 
     def close(self):
