@@ -315,13 +315,14 @@ struct DenseSplit {
     int cg;        // column groups of 64
     int s;         // splits of the contraction (1: C written directly)
     int s4_split;  // fragment groups per split
+    int s_work;    // splits (>= s) that the workspace of partial sums is sized for
 };
 DenseSplit dense_split(long long M, long long N, int K);
 // Position of A[r][n] (M x N) in the fragment order the GEMM reads (an array of
 // 16 ceil(M/16) x 16 ceil(N/16) floats, zero where r >= M or n >= N).
 long long dense_fragment_index(long long r, long long n, long long S4);
 // C = A B (optionally rows times row_scale), A in fragment order; work holds
-// dense_split(M, N, K).s * K * M floats when that split count exceeds 1.
+// dense_split(M, N, K).s * K * M floats when that split count exceeds 1 (plans hold s_work).
 int launch_dense_gemm(const float *Af, long long M, long long N, const float *B, long long ldb, int K, float *C,
                       long long ldc, const float *row_scale, float *work, void *stream);
 int launch_uv_from_vordiv(const DevPlan *P, int nharm, const void *vor, const void *div, void *U,

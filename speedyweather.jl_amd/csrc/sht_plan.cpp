@@ -1167,8 +1167,8 @@ static int build_matrices(sht_plan *pl) {
     long long work = 1;
     for (int K = 1; K <= pl->d.nlayers; ++K) {
         const sht::DenseSplit ds = sht::dense_split(np, 2 * nh, K), da = sht::dense_split(2 * nh, np, K);
-        if (ds.s > 1) work = std::max(work, (long long)ds.s * K * np);
-        if (da.s > 1) work = std::max(work, (long long)da.s * K * 2 * nh);
+        if (ds.s_work > 1) work = std::max(work, (long long)ds.s_work * K * np);
+        if (da.s_work > 1) work = std::max(work, (long long)da.s_work * K * 2 * nh);
     }
     pl->dense_bytes = ((size_t)work * 4 + 255) & ~(size_t)255;  // in each stream's scratch
     pl->device_bytes += (long long)bytes + np * 4 + work * 4;

@@ -118,14 +118,18 @@ int launch_scale_points(const float *scale, void *field, long long npoints, long
 // C[r, k] *= row_scale[r].  The dense transform's products have few columns (K layers) and
 // a large A that must be read once, so the GEMM runs on v_mfma_f32_16x16x4_f32 with A in
 // fragment order (dense_fragment_index: each wave's load of four K-steps is 1 KiB
-// contiguous) and is bound by reading A for K up to 32.  Workgroup = four waves, each one
-// 16-row tile, times a split of the contraction; the split's rows of B (all K columns, up
-// to 64 per column group) are staged in LDS 64 at a time (all of a thread's loads in flight
-// before its stores) and shared by the four row tiles, and each wave's A loads for the next
-// 64 rows are issued before the current ones' products.  With one split the result is stored directly; otherwise partial sums go to
-// W[s][k][r] and a second kernel adds them in a fixed order (no atomics, deterministic).
+// contiguous) and is bound by reading A.  Workgroup = four waves, each one 16-row tile, times a
+// split of the contraction; the split's rows of B (all K columns, up to 64 per column group)
+// are staged in LDS 64 at a time, double-buffered (one barrier per chunk), and shared by the
+// four row tiles.  A step issues the next chunk's B loads before its A loads, so storing B
+// waits for no A, and A stays in flight through the step's products.  T63 K=32 (188 MB of A
+// per direction), round trip: 144 us with one buffer, B loaded after A and 16-way bank
+// conflicts of the stores; 106 us so (3.6 TB/s; K=2: 94.5 -> 78.8 us, 4.8 TB/s).  With one
+// split the result is stored directly; otherwise partial sums go to W[s][k][r] and a second
+// kernel adds them in a fixed order (no atomics, deterministic).
 
 constexpr int kDenseChunk = 4;  // fragment groups (16 contraction values each) staged at once
+constexpr int kDenseMinGroups = 16;  // shortest split of the contraction, in fragment groups
 constexpr int kDenseCols = 64;  // columns of B per column group (four column tiles)
 
 template <int NCT>
@@ -134,8 +138,11 @@ __global__ __launch_bounds__(256) void dense_mfma_kernel(const float4 *__restric
                                                          long long ldb, int K, int s4_split, float *__restrict__ out_,
                                                          long long ldo, int direct,
                                                          const float *__restrict__ row_scale) {
-    constexpr int BST = 16 * NCT + 16;  // LDS row stride: the four lane groups' rows on distinct banks
-    __shared__ float Bs[kDenseChunk * 16][BST];
+    // LDS row stride (17 modulo 32): a wave stores 64 rows of one column to distinct banks, and
+    // the four lane groups read their rows of 16 columns from nearly disjoint ones
+    constexpr int BST = 16 * NCT + (NCT % 2 ? 1 : 17);
+    constexpr int CR = kDenseChunk * 16;  // rows of B staged per chunk
+    __shared__ float Bs[2][CR][BST];
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row = lane & 15, kg = lane >> 4;
     const long long rt = (long long)blockIdx.x * 4 + w;  // idle waves (rt >= RT) still stage and synchronise
@@ -145,57 +152,71 @@ __global__ __launch_bounds__(256) void dense_mfma_kernel(const float4 *__restric
     const SHT_GLOBAL float *B = as_global(B_) + (long long)k0 * ldb;
     const SHT_GLOBAL fv4 *Aw = reinterpret_cast<const SHT_GLOBAL fv4 *>(as_global(Af_)) +
                                (min(rt, RT - 1) * S4) * 64 + lane;
-    f4 acc[NCT];
+    f4 acc[NCT], sum[NCT];
 #pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) acc[ct] = f4{0.f, 0.f, 0.f, 0.f};
-    // B staging: thread t takes rows q = (t + 256 u) % 128 of column j = (t + 256 u) / 128,
-    // all loads of a chunk in flight before its LDS stores
-    constexpr int CR = kDenseChunk * 16;                // rows staged per chunk
-    constexpr int PER = CR * 16 * NCT / 256;            // B values per thread and chunk
-    // this wave's A fragments: the next chunk's loads are issued before the current
-    // chunk's products (two register sets)
-    fv4 a0[kDenseChunk], a1[kDenseChunk];
-    auto load_a = [&](fv4 (&a)[kDenseChunk], long long c0) {
-        const long long nch = min((long long)kDenseChunk, s4b - c0);
+    for (int ct = 0; ct < NCT; ++ct) acc[ct] = sum[ct] = f4{0.f, 0.f, 0.f, 0.f};
+    // every 256 contraction values the running sum moves on (blocked summation: the longer
+    // splits of fewer workgroups would otherwise lose accuracy)
+    auto fold = [&]() {
 #pragma unroll
-        for (int c = 0; c < kDenseChunk; ++c) a[c] = Aw[(c0 + min((long long)c, nch - 1)) * 64];
+        for (int ct = 0; ct < NCT; ++ct) {
+            sum[ct] += acc[ct];
+            acc[ct] = f4{0.f, 0.f, 0.f, 0.f};
+        }
     };
-    auto chunk = [&](const fv4 (&a)[kDenseChunk], long long c0) {
-        const int nch = (int)min((long long)kDenseChunk, s4b - c0);
-        float bv[PER];
+    // Chunks of kDenseChunk fragment groups.  Step c stores the staged rows of B into LDS
+    // buffer c % 2, issues the loads of B and A of chunk c + 1 (B first: the next step waits
+    // for it while A is still in flight), synchronises once and multiplies.  Loads past the
+    // split re-read its last group (of A) or row 0 (of B, stored as zero).
+    constexpr int PER = CR * 16 * NCT / 256;  // B values per thread and chunk
+    const int nch = (int)((s4b - s4a + kDenseChunk - 1) / kDenseChunk);
+    const long long nmax = min(16 * s4b, N);
+    static_assert(CR == 64, "a lane stages one row of a chunk");
+    struct Ops {
+        fv4 a[kDenseChunk];
+        float b[PER];
+    };
+    auto load = [&](Ops &S, int c) {
+        c = min(c, nch - 1);
+        const long long c0 = s4a + (long long)c * kDenseChunk;
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {  // row lane of the chunk, column w + 4 u (uniform per wave)
+            const SHT_GLOBAL float *col = B + (long long)min(w + 4 * u, Kg - 1) * ldb;
+            S.b[u] = col[(unsigned)(16 * c0 + lane < nmax ? (int)(16 * c0) + lane : 0)];
+        }
+#pragma unroll
+        for (int v = 0; v < kDenseChunk; ++v) S.a[v] = Aw[(unsigned)min((int)c0 + v, (int)s4b - 1) * 64u];
+    };
+    auto step = [&](Ops &cur, Ops &nxt, int c) {
+        const long long c0 = s4a + (long long)c * kDenseChunk;
+        float (*bs)[BST] = Bs[c & 1];
 #pragma unroll
         for (int u = 0; u < PER; ++u) {
-            const int i = tid + 256 * u, q = i % CR, j = i / CR;
-            const long long n = 16 * c0 + q;
-            bv[u] = (q < 16 * nch && n < N && j < Kg) ? B[n + (long long)j * ldb] : 0.f;
+            const int j = w + 4 * u;
+            bs[lane][j] = 16 * c0 + lane < nmax && j < Kg ? cur.b[u] : 0.f;
         }
-        __syncthreads();  // the previous chunk's B is no longer read
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int i = tid + 256 * u;
-            Bs[i % CR][i / CR] = bv[u];
-        }
+        load(nxt, c + 1);
         __syncthreads();
 #pragma unroll
-        for (int c = 0; c < kDenseChunk; ++c) {
-            if (c >= nch) break;  // uniform
+        for (int v = 0; v < kDenseChunk; ++v) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int q = 16 * c + 4 * v + kg;
+            for (int k = 0; k < 4; ++k) {
+                const int q = 16 * v + 4 * k + kg;
 #pragma unroll
-                for (int ct = 0; ct < NCT; ++ct) acc[ct] = mfma_f32(a[c][v], Bs[q][ct * 16 + row], acc[ct]);
+                for (int ct = 0; ct < NCT; ++ct) acc[ct] = mfma_f32(cur.a[v][k], bs[q][ct * 16 + row], acc[ct]);
             }
         }
     };
-    long long c0 = s4a;
-    if (c0 < s4b) load_a(a0, c0);
-    for (; c0 < s4b; c0 += 2 * kDenseChunk) {  // uniform; straight-line body, each set waits for its own loads
-        if (c0 + kDenseChunk < s4b) load_a(a1, c0 + kDenseChunk);
-        chunk(a0, c0);
-        if (c0 + kDenseChunk >= s4b) break;
-        if (c0 + 2 * kDenseChunk < s4b) load_a(a0, c0 + 2 * kDenseChunk);
-        chunk(a1, c0 + kDenseChunk);
+    Ops S0, S1;
+    load(S0, 0);
+    int c = 0;
+    for (; c + 1 < nch; c += 2) {  // straight-line body: each set waits for its own loads
+        step(S0, S1, c);
+        step(S1, S0, c + 1);
+        if (c & 2) fold();
     }
+    if (c < nch) step(S0, S1, c);
+    fold();
     if (rt >= RT) return;
     SHT_GLOBAL float *out = as_global(out_);
 #pragma unroll
@@ -207,9 +228,9 @@ __global__ __launch_bounds__(256) void dense_mfma_kernel(const float4 *__restric
             const long long r = rt * 16 + 4 * kg + i;
             if (r >= M) continue;
             if (direct)
-                out[r + (long long)(k0 + k) * ldo] = acc[ct][i] * (row_scale ? as_global(row_scale)[r] : 1.f);
+                out[r + (long long)(k0 + k) * ldo] = sum[ct][i] * (row_scale ? as_global(row_scale)[r] : 1.f);
             else
-                out[((long long)sp * K + k0 + k) * M + r] = acc[ct][i];
+                out[((long long)sp * K + k0 + k) * M + r] = sum[ct][i];
         }
     }
 }
@@ -246,10 +267,18 @@ DenseSplit dense_split(long long M, long long N, int K) {
     d.s4 = (N + 15) / 16;
     d.cg = (K + kDenseCols - 1) / kDenseCols;
     const long long wgs = (d.rt + 3) / 4 * d.cg;
-    long long s = (2048 + wgs - 1) / wgs;  // about 2048 workgroups
-    s = std::max(1LL, std::min(s, d.s4));
-    d.s4_split = (int)((d.s4 + s - 1) / s);
-    d.s = (int)((d.s4 + d.s4_split - 1) / d.s4_split);  // every split non-empty
+    // About 1024 workgroups (four per CU resident), but at least kDenseMinGroups groups per
+    // split: shorter ones spend their time on partial sums (T31 K=32, round trip: 21.7 us with
+    // 16 groups, 43.8 with 2; T63 K=32: 106.7 us with 1024 workgroups, 110.5 with 2048, 118.1
+    // with 3072).
+    auto splits = [&](long long want, int &per) {  // of at least `want` equal parts, none empty
+        want = std::max(1LL, std::min(want, d.s4));
+        per = (int)((d.s4 + want - 1) / want);
+        return (int)((d.s4 + per - 1) / per);
+    };
+    d.s = splits(std::min((1024 + wgs - 1) / wgs, d.s4 / kDenseMinGroups), d.s4_split);
+    int per;
+    d.s_work = splits((2048 + wgs - 1) / wgs, per);  // callers' scratch limits count on this size
     return d;
 }
 
