@@ -224,45 +224,69 @@ struct PassCols {
     static constexpr int MAXI = (kFFTMaxRing / R * NCG + kFFTThreads - 1) / kFFTThreads;
 };
 
-template <int R, bool INV>
-__device__ void fft_subpass_wg(float2 *buf, const float2 *tw, int N, const FFTPass &pd, int tid) {
-    constexpr int CB = PassCols<R>::CB, NCG = PassCols<R>::NCG, MAXI = PassCols<R>::MAXI;
-    const int M = pd.M, l = pd.l;
-    const int nb = N / R;  // butterflies per column
-    const int items = nb * NCG;
-    const FastDiv divM(M, pd.mulM);
-    // item -> (column group, butterfly), NCG <= 4
-    auto split = [&](int it, int &cg, int &t) {
+// The rings of a workgroup's columns in the grid: northern ring fn, southern ring fs of the
+// first column, columns ld apart, ncol of them.
+struct GridRings {
+    SHT_GLOBAL float *fn, *fs;
+    long long ld;
+    int ncol;
+};
+
+// Twiddles of a ring on their way to LDS: loaded together with the ring's data (one memory
+// latency for both), stored after every load of the thread is in flight.
+struct Twiddles {
+    static constexpr int U = (kFFTMaxRing + kFFTThreads - 1) / kFFTThreads;
+    float2 v[U];
+    __device__ __forceinline__ void load(const float *twiddle, long long tw_off, int N, int tid) {
+        const SHT_GLOBAL float2 *g = as_global(reinterpret_cast<const float2 *>(twiddle)) + tw_off;
+#pragma unroll
+        for (int q = 0; q < U; ++q) v[q] = gload(g + (unsigned)min(q * kFFTThreads + tid, N - 1));
+    }
+    __device__ __forceinline__ void store(float2 *tw, int N, int tid) const {
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const int i = q * kFFTThreads + tid;
+            if (i < N) tw[i] = v[q];
+        }
+    }
+};
+
+// The work items of a (sub-)pass: item it = tid + kFFTThreads i is butterfly t of column group
+// cg; butterfly t = (b, u) reads points b + M (q + R u), q < R, of its columns.
+template <int R>
+struct PassItem {
+    int cg, u, b;
+    __device__ __forceinline__ PassItem(int it, int nb, const FastDiv &divM) {
         cg = 0;
 #pragma unroll
-        for (int k = 1; k < NCG; ++k) cg += it >= k * nb ? 1 : 0;
-        t = it - cg * nb;
-    };
+        for (int k = 1; k < PassCols<R>::NCG; ++k) cg += it >= k * nb ? 1 : 0;  // NCG <= 4
+        const int t = it - cg * nb;
+        u = divM.div(t);
+        b = t - u * divM.d;
+    }
+};
+
+// Butterflies of one thread's items in registers.
+template <int R, bool INV>
+struct PassRegs {
+    static constexpr int CB = PassCols<R>::CB, NCG = PassCols<R>::NCG, MAXI = PassCols<R>::MAXI;
     float2 a[MAXI][CB][R];
+    __device__ __forceinline__ void read(const float2 *buf, int N, const FFTPass &pd, int tid) {
+        const int M = pd.M, nb = N / R, items = nb * NCG;
+        const FastDiv divM(M, pd.mulM);
 #pragma unroll
-    for (int i = 0; i < MAXI; ++i) {
-        const int it = tid + kFFTThreads * i;
-        if (it < items) {
-            int cg, t;
-            split(it, cg, t);
-            const int u = divM.div(t), b = t - u * M;
-            const float2 *src = buf + cg * CB * N + b + M * R * u;
+        for (int i = 0; i < MAXI; ++i) {
+            const int it = tid + kFFTThreads * i;
+            if (it >= items) continue;
+            const PassItem<R> p(it, nb, divM);
+            const float2 *src = buf + p.cg * CB * N + p.b + M * R * p.u;
 #pragma unroll
             for (int cc = 0; cc < CB; ++cc)
 #pragma unroll
                 for (int q = 0; q < R; ++q) a[i][cc][q] = src[cc * N + M * q];
         }
     }
-    __syncthreads();
-    const int ls = M * l;  // output stride between s
-    const int stepR = N / R;
-#pragma unroll
-    for (int i = 0; i < MAXI; ++i) {
-        const int it = tid + kFFTThreads * i;
-        if (it >= items) continue;
-        int cg, t;
-        split(it, cg, t);
-        const int u = divM.div(t), b = t - u * M;
+    __device__ __forceinline__ void butterflies(int i, int u, const float2 *tw, int stepR, int M) {
         if (u > 0) {
 #pragma unroll
             for (int q = 1; q < R; ++q) {
@@ -271,13 +295,32 @@ __device__ void fft_subpass_wg(float2 *buf, const float2 *tw, int N, const FFTPa
                 for (int cc = 0; cc < CB; ++cc) a[i][cc][q] = cmul(a[i][cc][q], w);
             }
         }
-        float2 *dst = buf + cg * CB * N + b + M * u;
 #pragma unroll
-        for (int cc = 0; cc < CB; ++cc) {
-            bfly_any<R, INV>(a[i][cc], tw, stepR);
+        for (int cc = 0; cc < CB; ++cc) bfly_any<R, INV>(a[i][cc], tw, stepR);
+    }
+};
+
+template <int R, bool INV>
+__device__ void fft_subpass_wg(float2 *buf, const float2 *tw, int N, const FFTPass &pd, int tid) {
+    typedef PassRegs<R, INV> Regs;
+    constexpr int CB = Regs::CB;
+    const int M = pd.M, nb = N / R, items = nb * Regs::NCG;
+    const FastDiv divM(M, pd.mulM);
+    Regs x;
+    x.read(buf, N, pd, tid);
+    __syncthreads();
+    const int ls = M * pd.l;  // output stride between s
 #pragma unroll
-            for (int s = 0; s < R; ++s) dst[cc * N + ls * s] = a[i][cc][s];
-        }
+    for (int i = 0; i < Regs::MAXI; ++i) {
+        const int it = tid + kFFTThreads * i;
+        if (it >= items) continue;
+        const PassItem<R> p(it, nb, divM);
+        x.butterflies(i, p.u, tw, N / R, pd.M);
+        float2 *dst = buf + p.cg * CB * N + p.b + M * p.u;
+#pragma unroll
+        for (int cc = 0; cc < CB; ++cc)
+#pragma unroll
+            for (int s = 0; s < R; ++s) dst[cc * N + ls * s] = x.a[i][cc][s];
     }
     __syncthreads();
 }
@@ -287,6 +330,40 @@ __device__ void fft_pass_wg(float2 *buf, const float2 *tw, int N, const FFTPass 
 #pragma unroll
     for (int sp = 0; sp < PassCols<R>::SUB; ++sp)
         fft_subpass_wg<R, INV>(buf + sp * (kFFTCols / PassCols<R>::SUB) * N, tw, N, pd, tid);
+}
+
+// Last pass (M = 1, u = t) with its results stored straight to the grid: point u + l s of a
+// butterfly's columns, so neighbouring lanes store neighbouring points.
+template <int R, bool INV>
+__device__ void fft_last_pass(const float2 *buf, const float2 *tw, int N, const FFTPass &pd, const GridRings &out,
+                              int tid) {
+    typedef PassRegs<R, INV> Regs;
+    constexpr int CB = Regs::CB, SC = kFFTCols / PassCols<R>::SUB;
+    const int nb = N / R, items = nb * Regs::NCG;
+    const FastDiv divM(1, 0u);
+#pragma unroll
+    for (int sp = 0; sp < PassCols<R>::SUB; ++sp) {
+        Regs x;
+        x.read(buf + sp * SC * N, N, pd, tid);
+#pragma unroll
+        for (int i = 0; i < Regs::MAXI; ++i) {
+            const int it = tid + kFFTThreads * i;
+            if (it >= items) continue;
+            const PassItem<R> p(it, nb, divM);
+            x.butterflies(i, p.u, tw, N / R, pd.M);
+#pragma unroll
+            for (int cc = 0; cc < CB; ++cc) {
+                const int c = sp * SC + p.cg * CB + cc;
+                if (c >= out.ncol) continue;
+                SHT_GLOBAL float *fn = out.fn + c * out.ld + p.u, *fs = out.fs + c * out.ld + p.u;
+#pragma unroll
+                for (int s = 0; s < R; ++s) {
+                    fn[(unsigned)(nb * s)] = x.a[i][cc][s].x;
+                    fs[(unsigned)(nb * s)] = x.a[i][cc][s].y;
+                }
+            }
+        }
+    }
 }
 
 // First pass (l = 1) of an odd prime radix r >= 11 as two small GEMMs on MFMA, in place.
@@ -311,16 +388,27 @@ __device__ void fft_pass_wg(float2 *buf, const float2 *tw, int N, const FFTPass 
 // (a butterfly's outputs overwrite its inputs, which the other row tiles still read).
 // tmax: the last pair t with nonzero inputs (a synthesis reads only the orders m <= mt and
 // their mirrors N - m: x_t, x_{r-t} vanish for t > (mt + M - 1) / M); h otherwise.
+//
+// Pairs of values are rounded by one instruction per part (v_cvt_pk_bf16_f32) and widened
+// again by a shift or a mask.
 __device__ inline void split3_bf16(const float (&x)[8], b8 &hi, b8 &mid, b8 &lo) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    u4 part[3];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const __bf16 h = (__bf16)x[e];
-        const float r1 = x[e] - (float)h;  // exact
-        const __bf16 m = (__bf16)r1;
-        hi[e] = h;
-        mid[e] = m;
-        lo[e] = (__bf16)(r1 - (float)m);
+    for (int e = 0; e < 4; ++e) {
+        float a = x[2 * e], b = x[2 * e + 1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const unsigned v = __builtin_bit_cast(unsigned, b2{(__bf16)a, (__bf16)b});
+            part[q][e] = v;
+            a -= __uint_as_float(v << 16);  // exact
+            b -= __uint_as_float(v & 0xFFFF0000u);
+        }
     }
+    hi = __builtin_bit_cast(b8, part[0]);
+    mid = __builtin_bit_cast(b8, part[1]);
+    lo = __builtin_bit_cast(b8, part[2]);
 }
 
 // c += a b over the parts (i, j) with i + j <= 2, smallest first
@@ -369,16 +457,17 @@ __device__ void fft_pass_mfma_first(float2 *buf, const SHT_GLOBAL b8 *tab, int N
                 ob = base;
                 z0 = buf[base];  // x_0, read before any output of the round is written
             }
+            // t past h re-reads the pair h, for which the table holds zeros; pairs between tmax and
+            // h are zero themselves
+            const float *pa = bf + 2 * base + ri, *pb = pa + 2 * M * r;
             for (int kc = 0; kc < KU; ++kc) {
                 float xs[8], xd[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const int t = 32 * kc + 8 * grp + e + 1;
-                    const bool ok = t <= tmax;
-                    const int tt = ok ? t : tmax;
-                    const float xa = bf[2 * (base + M * tt) + ri], xb = bf[2 * (base + M * (r - tt)) + ri];
-                    xs[e] = ok ? xa + xb : 0.f;
-                    xd[e] = ok ? xa - xb : 0.f;
+                    const int o = __mul24(min(32 * kc + 8 * grp + e + 1, h), 2 * M);
+                    const float xa = pa[o], xb = pb[-o];
+                    xs[e] = xa + xb;
+                    xd[e] = xa - xb;
                 }
                 b8 sh, sm, sl, dh, dm, dl;
                 split3_bf16(xs, sh, sm, sl);
@@ -386,10 +475,10 @@ __device__ void fft_pass_mfma_first(float2 *buf, const SHT_GLOBAL b8 *tab, int N
 #pragma unroll
                 for (int i = 0; i < kPrimeRowTiles; ++i) {
                     if (i >= nrt) break;  // uniform per wave
-                    const SHT_GLOBAL b8 *a = tab + ((long long)((r0 + i * G) * KC + kc) * 64 + lane) * 6;
-                    const b8 ch = a[0], cm = a[1], cl = a[2];
+                    const SHT_GLOBAL b8 *a = tab + ((r0 + i * G) * KC + kc) * 384 + lane;
+                    const b8 ch = a[0], cm = a[64], cl = a[128];
                     t1[i] = mma_bf16x3(ch, cm, cl, sh, sm, sl, t1[i]);
-                    const b8 nh = a[3], nm = a[4], nl = a[5];
+                    const b8 nh = a[192], nm = a[256], nl = a[320];
                     t2[i] = mma_bf16x3(nh, nm, nl, dh, dm, dl, t2[i]);
                 }
             }
@@ -435,10 +524,19 @@ __device__ __forceinline__ FFTPass load_pass(const SHT_GLOBAL FFTPass *p) {
 }
 
 // Runs all passes in place on buf (kFFTCols columns of N points, the first ncol of them
-// data): a first-pass MFMA radix, then the register passes, all across the workgroup.
-template <bool INV>
-__device__ __attribute__((always_inline)) void fft_run(const DevPlan &P, const FFTRing &R, float2 *buf,
-                                                        const float2 *tw, int N, int mt, int ncol, int tid) {
+// data): a first-pass MFMA radix, then the register passes (pd: the first one's descriptor), all across the workgroup.  Every pass ends with a barrier.
+// The plan tables the FFT kernels read, fetched with the ring record (one level of scalar
+// loads), and the first register pass's descriptor, fetched before the ring's data.
+struct FFTPlanTables {
+    const float *twiddle;
+    const FFTPass *passes;
+    const unsigned short *prime_tab;
+};
+
+template <bool INV, bool LAST>
+__device__ __attribute__((always_inline)) void fft_run(const FFTPlanTables &P, const FFTRing &R, float2 *buf,
+                                                        const float2 *tw, int N, int mt, int ncol, FFTPass pd,
+                                                        const GridRings &out, int tid) {
     const SHT_GLOBAL FFTPass *passes = as_global(P.passes) + R.passes;
     const int nf = R.nf;
     int f = 0;
@@ -455,8 +553,9 @@ __device__ __attribute__((always_inline)) void fft_run(const DevPlan &P, const F
         fft_pass_mfma_first<INV>(buf, tab, N, p0, ncol, max(tmax, 1), tid);
         f = 1;
     }
-    for (int g = f; g < nf; ++g) {
-        const FFTPass pd = load_pass(passes + g);
+    for (int g = f; g < nf - (LAST ? 1 : 0); ++g) {
+        // the next pass's descriptor loads while this one runs (past the last: its own again)
+        const FFTPass nx = load_pass(passes + min(g + 1, nf - 1));
         switch (pd.R) {
             case 16: fft_pass_wg<16, INV>(buf, tw, N, pd, tid); break;
             case 8: fft_pass_wg<8, INV>(buf, tw, N, pd, tid); break;
@@ -468,24 +567,20 @@ __device__ __attribute__((always_inline)) void fft_run(const DevPlan &P, const F
             case 11: fft_pass_wg<11, INV>(buf, tw, N, pd, tid); break;
             default: fft_pass_wg<13, INV>(buf, tw, N, pd, tid); break;  // the plan admits no other radix
         }
+        pd = nx;
     }
-}
-
-// Twiddles of ring j into LDS with all loads of a thread in flight together.
-__device__ inline void load_twiddles(const DevPlan &P, long long tw_off, int N, float2 *tw, int tid) {
-    const SHT_GLOBAL float2 *gtw = as_global(reinterpret_cast<const float2 *>(P.twiddle)) + tw_off;
-    constexpr int U = (kFFTMaxRing + kFFTThreads - 1) / kFFTThreads;
-    float2 v[U];
-#pragma unroll
-    for (int q = 0; q < U; ++q) {
-        const int i = q * kFFTThreads + tid;
-        if (i < N) v[q] = gload(gtw + i);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // every load in flight before the first LDS store
-#pragma unroll
-    for (int q = 0; q < U; ++q) {
-        const int i = q * kFFTThreads + tid;
-        if (i < N) tw[i] = v[q];
+    if constexpr (LAST) {
+        switch (pd.R) {
+            case 16: fft_last_pass<16, INV>(buf, tw, N, pd, out, tid); break;
+            case 8: fft_last_pass<8, INV>(buf, tw, N, pd, out, tid); break;
+            case 2: fft_last_pass<2, INV>(buf, tw, N, pd, out, tid); break;
+            case 3: fft_last_pass<3, INV>(buf, tw, N, pd, out, tid); break;
+            case 4: fft_last_pass<4, INV>(buf, tw, N, pd, out, tid); break;
+            case 5: fft_last_pass<5, INV>(buf, tw, N, pd, out, tid); break;
+            case 7: fft_last_pass<7, INV>(buf, tw, N, pd, out, tid); break;
+            case 11: fft_last_pass<11, INV>(buf, tw, N, pd, out, tid); break;
+            default: fft_last_pass<13, INV>(buf, tw, N, pd, out, tid); break;
+        }
     }
 }
 
@@ -526,15 +621,15 @@ struct FFTTile {
 // back to back on the same XCD: block b -> XCD b % 8, slot s = b / 8, unit
 // (s / 2) * 8 + b % 8, column group 2 p + s % 2.  Otherwise (analysis): block b -> ring
 // rank b / kgs, column group b % kgs.  Batch tiles carry the rank (m) and column group.
-// rings: the plan's ring records (single calls pass them in place of a tile list).
-// Returns false for blocks past the end.
+// rings: the plan's ring records (single calls pass them in place of a tile list), followed by
+// copies of the first marked j < 0 up to a multiple of the XCD count: blocks past the last ring
+// issue a valid ring's loads and then exit, so that no branch stands between the kernel's
+// arguments and the loads that depend on them.
 template <bool BATCH>
-__device__ inline bool fft_tile(const DevPlan &P, const SHT_GLOBAL FFTRing *rings, const Tile &T, int K, bool paired,
-                                FFTTile &t) {
+__device__ inline void fft_tile(const SHT_GLOBAL FFTRing *rings, const Tile &T, int K, bool paired, FFTTile &t) {
     const int kgs = (K + kFFTCols - 1) / kFFTCols;
     int cg, r;
     if (BATCH) {
-        if (T.m < 0) return false;
         r = T.m;
         cg = T.blk;
     } else {
@@ -550,12 +645,10 @@ __device__ inline bool fft_tile(const DevPlan &P, const SHT_GLOBAL FFTRing *ring
             r = b / kgs;
             cg = b - r * kgs;
         }
-        if (r >= P.n || cg >= kgs) return false;
     }
     t.R = load_ring(rings + r);
     t.k0 = cg * kFFTCols;
     t.ncol = min(kFFTCols, K - t.k0);
-    return true;
 }
 
 // Fourier rows are read and written with thread -> (order mm = tid/4 + 64 u, column tid%4).
@@ -575,18 +668,23 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
     extern __shared__ float2 smem[];
     const int tid = threadIdx.x;
     const Tile T = BATCH ? tiles[blockIdx.x] : Tile{0, 0, 0, 0};
+    if (BATCH && T.m < 0) return;  // padding of the launch order
     const CallArgs C = BATCH ? calls[T.call] : single;
     const DevPlan &P = plans[C.plan];
     const int K = C.K;
     const SHT_GLOBAL FFTRing *rings =
         BATCH ? as_global(P.rings) : as_global(reinterpret_cast<const FFTRing *>(tiles));
+    const FFTPlanTables tables{P.twiddle, P.passes, P.prime_tab};
     FFTTile G;
-    if (!fft_tile<BATCH>(P, rings, T, K, C.paired != 0, G)) return;  // padding of the launch order
+    fft_tile<BATCH>(rings, T, K, C.paired != 0, G);
     const FFTRing &R = G.R;
     const int N = R.N, mt = R.mt, ncol = G.ncol;
+    __builtin_assume(N >= 1 && N <= kFFTMaxRing);  // offsets within a ring fit scalar-base loads
     float2 *tw = smem;
     float2 *b0 = smem + N;
-    load_twiddles(P, R.tw_off, N, tw, tid);
+    const FFTPass pass0 = load_pass(as_global(tables.passes) + R.passes + (R.prime ? min(1, R.nf - 1) : 0));
+    Twiddles twr;
+    twr.load(tables.twiddle, R.tw_off, N, tid);
     {
         const SHT_GLOBAL float4 *fb =
             as_global(static_cast<const float4 *>(C.fbuf)) + R.fboff * (long long)K + G.k0;
@@ -599,7 +697,9 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
             v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (col < ncol && mm <= mt) v[u] = gload(fb + (unsigned)(mm * K + col));
         }
+        if (!BATCH && R.j < 0) return;
         __builtin_amdgcn_sched_barrier(0);  // every load in flight before the first LDS store
+        twr.store(tw, N, tid);
         if (C.adj) {  // adjoint of the analysis (grid2spec pullback): rows times ΔΩ_j / s_m
             const float wj = as_global(P.domega)[R.j];
 #pragma unroll
@@ -626,47 +726,32 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
         }
     }
     __syncthreads();
-    fft_run<true>(P, R, b0, tw, N, mt, ncol, tid);
-    __syncthreads();
-    {
-        SHT_GLOBAL float *field = as_global(static_cast<float *>(C.out));
-        const long long ld = C.ld_out;
-        const long long rn = R.ring_n, rs = R.ring_s;
+    SHT_GLOBAL float *field = as_global(static_cast<float *>(C.out)) + (long long)G.k0 * C.ld_out;
+    const GridRings out{field + R.ring_n, field + R.ring_s, C.ld_out, ncol};
+    fft_run<true, !ACC>(tables, R, b0, tw, N, mt, ncol, pass0, out, tid);
+    if constexpr (ACC) {
+        // pullback: add into the caller's cotangent; a column's old values are all read before
+        // its first store, so the reads are in flight together
         constexpr int U = (kFFTMaxRing + kFFTThreads - 1) / kFFTThreads;
 #pragma unroll
         for (int c = 0; c < kFFTCols; ++c) {
             if (c >= ncol) break;  // uniform
-            SHT_GLOBAL float *fn = field + (long long)(G.k0 + c) * ld + rn;
-            SHT_GLOBAL float *fs = field + (long long)(G.k0 + c) * ld + rs;
+            SHT_GLOBAL float *fn = out.fn + c * out.ld, *fs = out.fs + c * out.ld;
             const float2 *z = b0 + c * N;
-            if constexpr (ACC) {
-                // pullback: add into the caller's cotangent; the column's old values are all
-                // read before its first store, so the reads are in flight together
-                float on[U], os[U];
+            float on[U], os[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int i = min(u * kFFTThreads + tid, N - 1);
-                    on[u] = fn[(unsigned)i];
-                    os[u] = fs[(unsigned)i];
-                }
+            for (int u = 0; u < U; ++u) {
+                const int i = min(u * kFFTThreads + tid, N - 1);
+                on[u] = fn[(unsigned)i];
+                os[u] = fs[(unsigned)i];
+            }
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int i = u * kFFTThreads + tid;
-                    if (i < N) {
-                        const float2 v = z[i];
-                        fn[(unsigned)i] = on[u] + v.x;
-                        fs[(unsigned)i] = os[u] + v.y;
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int i = u * kFFTThreads + tid;
-                    if (i < N) {
-                        const float2 v = z[i];
-                        fn[(unsigned)i] = v.x;
-                        fs[(unsigned)i] = v.y;
-                    }
+            for (int u = 0; u < U; ++u) {
+                const int i = u * kFFTThreads + tid;
+                if (i < N) {
+                    const float2 v = z[i];
+                    fn[(unsigned)i] = on[u] + v.x;
+                    fs[(unsigned)i] = os[u] + v.y;
                 }
             }
         }
@@ -684,31 +769,35 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
     extern __shared__ float2 smem[];
     const int tid = threadIdx.x;
     const Tile T = BATCH ? tiles[blockIdx.x] : Tile{0, 0, 0, 0};
+    if (BATCH && T.m < 0) return;  // padding of the launch order
     const CallArgs C = BATCH ? calls[T.call] : single;
     const DevPlan &P = plans[C.plan];
     const int K = C.K;
     const SHT_GLOBAL FFTRing *rings =
         BATCH ? as_global(P.rings) : as_global(reinterpret_cast<const FFTRing *>(tiles));
+    const FFTPlanTables tables{P.twiddle, P.passes, P.prime_tab};
     FFTTile G;
-    if (!fft_tile<BATCH>(P, rings, T, K, false, G)) return;  // padding of the launch order
+    fft_tile<BATCH>(rings, T, K, false, G);
     const FFTRing &R = G.R;
     const int N = R.N, mt = R.mt, ncol = G.ncol;
+    __builtin_assume(N >= 1 && N <= kFFTMaxRing);  // offsets within a ring fit scalar-base loads
     float2 *tw = smem;
     float2 *b0 = smem + N;
-    load_twiddles(P, R.tw_off, N, tw, tid);
+    const FFTPass pass0 = load_pass(as_global(tables.passes) + R.passes + (R.prime ? min(1, R.nf - 1) : 0));
+    Twiddles twr;
+    twr.load(tables.twiddle, R.tw_off, N, tid);
+    const SHT_GLOBAL float *field = as_global(static_cast<const float *>(C.in)) + (long long)G.k0 * C.ld_in;
+    const GridRings in{const_cast<SHT_GLOBAL float *>(field + R.ring_n), const_cast<SHT_GLOBAL float *>(field + R.ring_s),
+                       C.ld_in, ncol};
     {
-        const SHT_GLOBAL float *field = as_global(static_cast<const float *>(C.in));
-        const long long ld = C.ld_in;
-        const long long rn = R.ring_n, rs = R.ring_s;
         constexpr int U = (kFFTMaxRing + kFFTThreads - 1) / kFFTThreads;
         // all loads of the thread in flight before the first LDS store (columns past ncol
         // re-read column 0 and are not stored)
         float vn[kFFTCols][U], vs[kFFTCols][U];
 #pragma unroll
         for (int c = 0; c < kFFTCols; ++c) {
-            const int cc = c < ncol ? c : 0;
-            const SHT_GLOBAL float *fn = field + (long long)(G.k0 + cc) * ld + rn;
-            const SHT_GLOBAL float *fs = field + (long long)(G.k0 + cc) * ld + rs;
+            const long long o = (long long)(c < ncol ? c : 0) * in.ld;
+            const SHT_GLOBAL float *fn = in.fn + o, *fs = in.fs + o;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const unsigned i = min(u * kFFTThreads + tid, N - 1);
@@ -717,6 +806,7 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
             }
         }
         __builtin_amdgcn_sched_barrier(0);
+        twr.store(tw, N, tid);
 #pragma unroll
         for (int c = 0; c < kFFTCols; ++c) {
 #pragma unroll
@@ -725,10 +815,9 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
                 if (c < ncol && i < N) b0[c * N + i] = make_float2(vn[c][u], vs[c][u]);
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
-    fft_run<false>(P, R, b0, tw, N, mt, ncol, tid);
-    __syncthreads();
+    fft_run<false, false>(tables, R, b0, tw, N, mt, ncol, pass0, GridRings{}, tid);
     {
         SHT_GLOBAL float4 *fb = as_global(static_cast<float4 *>(C.fbuf)) + R.fboff * (long long)K + G.k0;
         const int col = tid % kFFTCols, m0 = tid / kFFTCols;

@@ -247,8 +247,8 @@ struct DevPlan {
     const int *nfac;
     // First-pass prime radices r (MFMA pass): per r, cos / sin(2 pi s t / r) for rows
     // s = 0..h (tiles of 16) and t = 1..h (chunks of 32), h = (r-1)/2, as three BF16 parts of
-    // the FP64 values in MFMA fragment order: per (row tile, chunk, lane) six vectors of 8
-    // (cos hi, mid, lo, sin hi, mid, lo).  prime_off[r] (r < 256): r's first vector.
+    // the FP64 values in MFMA fragment order: per (row tile, chunk) six fragments (cos hi, mid,
+    // lo, sin hi, mid, lo) of a vector of 8 per lane, 1 KiB contiguous each.  prime_off[r] (r < 256): r's first vector.
     const unsigned short *prime_tab;
     const long long *prime_off;
     // Ring DFT on MFMA (rings of N = 4p points): per ring, the cos / sin matrices

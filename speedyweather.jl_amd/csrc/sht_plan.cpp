@@ -588,15 +588,15 @@ void prime_tables(const std::vector<int> (&fac_v)[kPolicies], const std::vector<
                             v[0] = std::cos(a);
                             v[1] = std::sin(a);
                         }
-                        const size_t base = (size_t)8 * (off[r] + ((size_t)(mt * KC + kc) * 64 + lane) * 6) + e;
+                        const size_t base = (size_t)8 * (off[r] + (size_t)(mt * KC + kc) * 384 + lane) + e;
                         for (int cs = 0; cs < 2; ++cs) {
                             const uint16_t hi = to_bf16(v[cs]);
                             const double r1 = v[cs] - bf16_value(hi);
                             const uint16_t mid = to_bf16(r1);
                             const uint16_t lo = to_bf16(r1 - bf16_value(mid));
-                            tab[base + (size_t)(3 * cs + 0) * 8] = hi;
-                            tab[base + (size_t)(3 * cs + 1) * 8] = mid;
-                            tab[base + (size_t)(3 * cs + 2) * 8] = lo;
+                            tab[base + (size_t)(3 * cs + 0) * 512] = hi;
+                            tab[base + (size_t)(3 * cs + 1) * 512] = mid;
+                            tab[base + (size_t)(3 * cs + 2) * 512] = lo;
                         }
                     }
     }
@@ -1018,8 +1018,9 @@ int build_plan(sht_plan *pl) {
         for (int q = 0; q < kPolicies; ++q) {
             if (!pl->pol_ok[q]) continue;
             if ((rc = dev_upload(A, pl->h_ring_order_v[q], &views[q].ring_order))) return rc;
-            // the rings' records in launch order
-            std::vector<sht::FFTRing> rings(n);
+            // the rings' records in launch order, then copies of the first marked j < 0 for the
+            // launches whose ring ranks are padded to a multiple of the XCD count
+            std::vector<sht::FFTRing> rings((n + sht::kXCDs - 1) / sht::kXCDs * sht::kXCDs, sht::FFTRing{});
             for (int r = 0; r < n; ++r) {
                 const int j = pl->h_ring_order_v[q][r];
                 sht::FFTRing &x = rings[r];
@@ -1044,6 +1045,10 @@ int build_plan(sht_plan *pl) {
                 x.ring_n = g.ring_n[j];
                 x.ring_s = g.ring_s[j];
                 x.passes = (long long)j * sht::kMaxFactors;
+            }
+            for (size_t r = n; r < rings.size(); ++r) {
+                rings[r] = rings[0];
+                rings[r].j = -1;
             }
             if ((rc = dev_upload(A, rings, &views[q].rings))) return rc;
             if ((rc = dev_upload(A, pass_table(g, fac_v[q], nfac_v[q]), &views[q].passes))) return rc;
