@@ -213,16 +213,39 @@ __device__ inline void bfly_any(float2 *a, const float2 *tw, int stepR) {
 // thread reads all its items into registers, the workgroup synchronises, then the results
 // are written in place.  Columns past the call's last column hold scratch values that are
 // transformed along and never stored.
-// Radices 11 and 13 (one column per item) run as two sub-passes of two columns each, so
-// that a thread holds at most one butterfly; radix 16 (N / 16 butterflies per column, at
-// most 256 items over four columns) needs no split.
-template <int R>
+// CB by the number of butterflies per column (pass_columns): the fewest columns per item whose
+// items still fit the workgroup's threads at once, so that short rings use all four waves
+// instead of a few lanes with all columns each (T31 K=8: 5.7 -> 4.6 us synthesis, 5.8 -> 5.0
+// analysis; T127 K=32: 9.2 -> 8.8, 9.4 -> 9.2).
+// Radices 11 and 13 (one column per item) run as two sub-passes of two columns each where the
+// items of four columns exceed the threads.
+template <int R, int CBv, int SUBv = 1>
 struct PassCols {
-    static constexpr int CB = R <= 7 ? 4 : R <= 8 ? 2 : 1;  // columns per work item
-    static constexpr int SUB = R <= 8 || R == 16 ? 1 : 2;   // column sub-passes
-    static constexpr int NCG = kFFTCols / CB / SUB;         // column groups per sub-pass
-    static constexpr int MAXI = (kFFTMaxRing / R * NCG + kFFTThreads - 1) / kFFTThreads;
+    static constexpr int CB = CBv;                   // columns per work item
+    static constexpr int SUB = SUBv;                 // column sub-passes
+    static constexpr int NCG = kFFTCols / CB / SUB;  // column groups per sub-pass
+    static constexpr int kMaxB = kFFTMaxRing / R;    // butterflies per column
+    // the largest butterfly count this choice serves (pass_columns)
+    static constexpr int kMaxNb = CB == 1 && SUB == 1 ? 64 : kMaxB;
+    static constexpr int MAXI = ((kMaxNb < kMaxB ? kMaxNb : kMaxB) * NCG + kFFTThreads - 1) / kFFTThreads;
 };
+// Calls f with the column choice for nb butterflies per column.
+template <int R, class F>
+__device__ __forceinline__ void pass_columns(int nb, F &&f) {
+    if constexpr (R == 16) {  // nb <= 64
+        f(PassCols<R, 1>{});
+    } else if constexpr (R > 8) {
+        if (nb <= 64)
+            f(PassCols<R, 1>{});
+        else
+            f(PassCols<R, 1, 2>{});
+    } else {
+        if (nb <= 64)
+            f(PassCols<R, 1>{});
+        else
+            f(PassCols<R, 2>{});
+    }
+}
 
 // The rings of a workgroup's columns in the grid: northern ring fn, southern ring fs of the
 // first column, columns ld apart, ncol of them.
@@ -253,13 +276,13 @@ struct Twiddles {
 
 // The work items of a (sub-)pass: item it = tid + kFFTThreads i is butterfly t of column group
 // cg; butterfly t = (b, u) reads points b + M (q + R u), q < R, of its columns.
-template <int R>
+template <class PC>
 struct PassItem {
     int cg, u, b;
     __device__ __forceinline__ PassItem(int it, int nb, const FastDiv &divM) {
         cg = 0;
 #pragma unroll
-        for (int k = 1; k < PassCols<R>::NCG; ++k) cg += it >= k * nb ? 1 : 0;  // NCG <= 4
+        for (int k = 1; k < PC::NCG; ++k) cg += it >= k * nb ? 1 : 0;  // NCG <= 4
         const int t = it - cg * nb;
         u = divM.div(t);
         b = t - u * divM.d;
@@ -267,9 +290,9 @@ struct PassItem {
 };
 
 // Butterflies of one thread's items in registers.
-template <int R, bool INV>
+template <int R, bool INV, class PC>
 struct PassRegs {
-    static constexpr int CB = PassCols<R>::CB, NCG = PassCols<R>::NCG, MAXI = PassCols<R>::MAXI;
+    static constexpr int CB = PC::CB, NCG = PC::NCG, MAXI = PC::MAXI;
     float2 a[MAXI][CB][R];
     __device__ __forceinline__ void read(const float2 *buf, int N, const FFTPass &pd, int tid) {
         const int M = pd.M, nb = N / R, items = nb * NCG;
@@ -278,12 +301,40 @@ struct PassRegs {
         for (int i = 0; i < MAXI; ++i) {
             const int it = tid + kFFTThreads * i;
             if (it >= items) continue;
-            const PassItem<R> p(it, nb, divM);
+            const PassItem<PC> p(it, nb, divM);
             const float2 *src = buf + p.cg * CB * N + p.b + M * R * p.u;
 #pragma unroll
             for (int cc = 0; cc < CB; ++cc)
 #pragma unroll
                 for (int q = 0; q < R; ++q) a[i][cc][q] = src[cc * N + M * q];
+        }
+    }
+    // the last pass (M = 1): a butterfly's inputs are consecutive; even radices read them in
+    // pairs (16-byte aligned: rings have a multiple of 4 points), half the bank conflicts of
+    // single points R apart
+    __device__ __forceinline__ void read_last(const float2 *buf, int N, int tid) {
+        const int nb = N / R, items = nb * NCG;
+        const FastDiv one(1, 0u);
+#pragma unroll
+        for (int i = 0; i < MAXI; ++i) {
+            const int it = tid + kFFTThreads * i;
+            if (it >= items) continue;
+            const PassItem<PC> p(it, nb, one);
+#pragma unroll
+            for (int cc = 0; cc < CB; ++cc) {
+                const float2 *src = buf + (p.cg * CB + cc) * N + R * p.u;
+                if constexpr (R % 2 == 0) {
+#pragma unroll
+                    for (int q = 0; q < R; q += 2) {
+                        const float4 v = *reinterpret_cast<const float4 *>(src + q);
+                        a[i][cc][q] = make_float2(v.x, v.y);
+                        a[i][cc][q + 1] = make_float2(v.z, v.w);
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < R; ++q) a[i][cc][q] = src[q];
+                }
+            }
         }
     }
     __device__ __forceinline__ void butterflies(int i, int u, const float2 *tw, int stepR, int M) {
@@ -300,21 +351,21 @@ struct PassRegs {
     }
 };
 
-template <int R, bool INV>
-__device__ void fft_subpass_wg(float2 *buf, const float2 *tw, int N, const FFTPass &pd, int tid) {
-    typedef PassRegs<R, INV> Regs;
+template <int R, bool INV, class PC>
+__device__ __forceinline__ void fft_subpass_wg(float2 *buf, const float2 *tw, int N, const FFTPass &pd, int tid) {
+    typedef PassRegs<R, INV, PC> Regs;
     constexpr int CB = Regs::CB;
     const int M = pd.M, nb = N / R, items = nb * Regs::NCG;
     const FastDiv divM(M, pd.mulM);
     Regs x;
     x.read(buf, N, pd, tid);
     __syncthreads();
-    const int ls = M * pd.l;  // output stride between s
+    const int ls = nb;  // output stride between s: M l = N / R
 #pragma unroll
     for (int i = 0; i < Regs::MAXI; ++i) {
         const int it = tid + kFFTThreads * i;
         if (it >= items) continue;
-        const PassItem<R> p(it, nb, divM);
+        const PassItem<PC> p(it, nb, divM);
         x.butterflies(i, p.u, tw, N / R, pd.M);
         float2 *dst = buf + p.cg * CB * N + p.b + M * p.u;
 #pragma unroll
@@ -327,29 +378,32 @@ __device__ void fft_subpass_wg(float2 *buf, const float2 *tw, int N, const FFTPa
 
 template <int R, bool INV>
 __device__ void fft_pass_wg(float2 *buf, const float2 *tw, int N, const FFTPass &pd, int tid) {
+    pass_columns<R>(N / R, [&](auto pc) {
+        typedef decltype(pc) PC;
 #pragma unroll
-    for (int sp = 0; sp < PassCols<R>::SUB; ++sp)
-        fft_subpass_wg<R, INV>(buf + sp * (kFFTCols / PassCols<R>::SUB) * N, tw, N, pd, tid);
+        for (int sp = 0; sp < PC::SUB; ++sp)
+            fft_subpass_wg<R, INV, PC>(buf + sp * (kFFTCols / PC::SUB) * N, tw, N, pd, tid);
+    });
 }
 
 // Last pass (M = 1, u = t) with its results stored straight to the grid: point u + l s of a
 // butterfly's columns, so neighbouring lanes store neighbouring points.
-template <int R, bool INV>
-__device__ void fft_last_pass(const float2 *buf, const float2 *tw, int N, const FFTPass &pd, const GridRings &out,
-                              int tid) {
-    typedef PassRegs<R, INV> Regs;
-    constexpr int CB = Regs::CB, SC = kFFTCols / PassCols<R>::SUB;
+template <int R, bool INV, class PC>
+__device__ __forceinline__ void fft_last_columns(const float2 *buf, const float2 *tw, int N, const FFTPass &pd,
+                                                 const GridRings &out, int tid) {
+    typedef PassRegs<R, INV, PC> Regs;
+    constexpr int CB = Regs::CB, SC = kFFTCols / PC::SUB;
     const int nb = N / R, items = nb * Regs::NCG;
     const FastDiv divM(1, 0u);
 #pragma unroll
-    for (int sp = 0; sp < PassCols<R>::SUB; ++sp) {
+    for (int sp = 0; sp < PC::SUB; ++sp) {
         Regs x;
-        x.read(buf + sp * SC * N, N, pd, tid);
+        x.read_last(buf + sp * SC * N, N, tid);
 #pragma unroll
         for (int i = 0; i < Regs::MAXI; ++i) {
             const int it = tid + kFFTThreads * i;
             if (it >= items) continue;
-            const PassItem<R> p(it, nb, divM);
+            const PassItem<PC> p(it, nb, divM);
             x.butterflies(i, p.u, tw, N / R, pd.M);
 #pragma unroll
             for (int cc = 0; cc < CB; ++cc) {
@@ -364,6 +418,12 @@ __device__ void fft_last_pass(const float2 *buf, const float2 *tw, int N, const 
             }
         }
     }
+}
+
+template <int R, bool INV>
+__device__ void fft_last_pass(const float2 *buf, const float2 *tw, int N, const FFTPass &pd, const GridRings &out,
+                              int tid) {
+    pass_columns<R>(N / R, [&](auto pc) { fft_last_columns<R, INV, decltype(pc)>(buf, tw, N, pd, out, tid); });
 }
 
 // First pass (l = 1) of an odd prime radix r >= 11 as two small GEMMs on MFMA, in place.
@@ -550,36 +610,42 @@ __device__ __attribute__((always_inline)) void fft_run(const FFTPlanTables &P, c
         const SHT_GLOBAL b8 *tab = reinterpret_cast<const SHT_GLOBAL b8 *>(as_global(P.prime_tab)) + R.prime_off;
         const int h = (p0.R - 1) >> 1;
         const int tmax = INV ? min(h, (mt + p0.M - 1) / p0.M) : h;
-        fft_pass_mfma_first<INV>(buf, tab, N, p0, ncol, max(tmax, 1), tid);
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        fft_pass_mfma_first<INV>(buf, tab, N, p0, ncol, max(tmax, 1), t);
         f = 1;
     }
     for (int g = f; g < nf - (LAST ? 1 : 0); ++g) {
         // the next pass's descriptor loads while this one runs (past the last: its own again)
         const FFTPass nx = load_pass(passes + min(g + 1, nf - 1));
+        int t = tid;  // keeps every pass's index arithmetic inside the loop (hoisted, it spills)
+        asm volatile("" : "+v"(t));
         switch (pd.R) {
-            case 16: fft_pass_wg<16, INV>(buf, tw, N, pd, tid); break;
-            case 8: fft_pass_wg<8, INV>(buf, tw, N, pd, tid); break;
-            case 2: fft_pass_wg<2, INV>(buf, tw, N, pd, tid); break;
-            case 3: fft_pass_wg<3, INV>(buf, tw, N, pd, tid); break;
-            case 4: fft_pass_wg<4, INV>(buf, tw, N, pd, tid); break;
-            case 5: fft_pass_wg<5, INV>(buf, tw, N, pd, tid); break;
-            case 7: fft_pass_wg<7, INV>(buf, tw, N, pd, tid); break;
-            case 11: fft_pass_wg<11, INV>(buf, tw, N, pd, tid); break;
-            default: fft_pass_wg<13, INV>(buf, tw, N, pd, tid); break;  // the plan admits no other radix
+            case 16: fft_pass_wg<16, INV>(buf, tw, N, pd, t); break;
+            case 8: fft_pass_wg<8, INV>(buf, tw, N, pd, t); break;
+            case 2: fft_pass_wg<2, INV>(buf, tw, N, pd, t); break;
+            case 3: fft_pass_wg<3, INV>(buf, tw, N, pd, t); break;
+            case 4: fft_pass_wg<4, INV>(buf, tw, N, pd, t); break;
+            case 5: fft_pass_wg<5, INV>(buf, tw, N, pd, t); break;
+            case 7: fft_pass_wg<7, INV>(buf, tw, N, pd, t); break;
+            case 11: fft_pass_wg<11, INV>(buf, tw, N, pd, t); break;
+            default: fft_pass_wg<13, INV>(buf, tw, N, pd, t); break;  // the plan admits no other radix
         }
         pd = nx;
     }
     if constexpr (LAST) {
+        int t = tid;
+        asm volatile("" : "+v"(t));
         switch (pd.R) {
-            case 16: fft_last_pass<16, INV>(buf, tw, N, pd, out, tid); break;
-            case 8: fft_last_pass<8, INV>(buf, tw, N, pd, out, tid); break;
-            case 2: fft_last_pass<2, INV>(buf, tw, N, pd, out, tid); break;
-            case 3: fft_last_pass<3, INV>(buf, tw, N, pd, out, tid); break;
-            case 4: fft_last_pass<4, INV>(buf, tw, N, pd, out, tid); break;
-            case 5: fft_last_pass<5, INV>(buf, tw, N, pd, out, tid); break;
-            case 7: fft_last_pass<7, INV>(buf, tw, N, pd, out, tid); break;
-            case 11: fft_last_pass<11, INV>(buf, tw, N, pd, out, tid); break;
-            default: fft_last_pass<13, INV>(buf, tw, N, pd, out, tid); break;
+            case 16: fft_last_pass<16, INV>(buf, tw, N, pd, out, t); break;
+            case 8: fft_last_pass<8, INV>(buf, tw, N, pd, out, t); break;
+            case 2: fft_last_pass<2, INV>(buf, tw, N, pd, out, t); break;
+            case 3: fft_last_pass<3, INV>(buf, tw, N, pd, out, t); break;
+            case 4: fft_last_pass<4, INV>(buf, tw, N, pd, out, t); break;
+            case 5: fft_last_pass<5, INV>(buf, tw, N, pd, out, t); break;
+            case 7: fft_last_pass<7, INV>(buf, tw, N, pd, out, t); break;
+            case 11: fft_last_pass<11, INV>(buf, tw, N, pd, out, t); break;
+            default: fft_last_pass<13, INV>(buf, tw, N, pd, out, t); break;
         }
     }
 }
@@ -665,7 +731,8 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
                                                                     CallArgs single,
                                                                     const CallArgs *__restrict__ calls,
                                                                     const Tile *__restrict__ tiles) {
-    extern __shared__ float2 smem[];
+    extern __shared__ float4 smem4[];
+    float2 *smem = reinterpret_cast<float2 *>(smem4);
     const int tid = threadIdx.x;
     const Tile T = BATCH ? tiles[blockIdx.x] : Tile{0, 0, 0, 0};
     if (BATCH && T.m < 0) return;  // padding of the launch order
@@ -766,7 +833,8 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
                                                                    CallArgs single,
                                                                    const CallArgs *__restrict__ calls,
                                                                    const Tile *__restrict__ tiles) {
-    extern __shared__ float2 smem[];
+    extern __shared__ float4 smem4[];
+    float2 *smem = reinterpret_cast<float2 *>(smem4);
     const int tid = threadIdx.x;
     const Tile T = BATCH ? tiles[blockIdx.x] : Tile{0, 0, 0, 0};
     if (BATCH && T.m < 0) return;  // padding of the launch order
@@ -820,7 +888,9 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
     fft_run<false, false>(tables, R, b0, tw, N, mt, ncol, pass0, GridRings{}, tid);
     {
         SHT_GLOBAL float4 *fb = as_global(static_cast<float4 *>(C.fbuf)) + R.fboff * (long long)K + G.k0;
-        const int col = tid % kFFTCols, m0 = tid / kFFTCols;
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        const int col = t % kFFTCols, m0 = t / kFFTCols;
         const float2 *z = b0 + col * N;
         // adjoint of the synthesis (spec2grid pullback): rows times s_m (1/cos lat) / ΔΩ_j
         const float wj = C.adj ? (C.unscale ? as_global(P.coslat_inv)[R.j] : 1.f) / as_global(P.domega)[R.j] : 1.f;
