@@ -309,34 +309,6 @@ struct PassRegs {
                 for (int q = 0; q < R; ++q) a[i][cc][q] = src[cc * N + M * q];
         }
     }
-    // the last pass (M = 1): a butterfly's inputs are consecutive; even radices read them in
-    // pairs (16-byte aligned: rings have a multiple of 4 points), half the bank conflicts of
-    // single points R apart
-    __device__ __forceinline__ void read_last(const float2 *buf, int N, int tid) {
-        const int nb = N / R, items = nb * NCG;
-        const FastDiv one(1, 0u);
-#pragma unroll
-        for (int i = 0; i < MAXI; ++i) {
-            const int it = tid + kFFTThreads * i;
-            if (it >= items) continue;
-            const PassItem<PC> p(it, nb, one);
-#pragma unroll
-            for (int cc = 0; cc < CB; ++cc) {
-                const float2 *src = buf + (p.cg * CB + cc) * N + R * p.u;
-                if constexpr (R % 2 == 0) {
-#pragma unroll
-                    for (int q = 0; q < R; q += 2) {
-                        const float4 v = *reinterpret_cast<const float4 *>(src + q);
-                        a[i][cc][q] = make_float2(v.x, v.y);
-                        a[i][cc][q + 1] = make_float2(v.z, v.w);
-                    }
-                } else {
-#pragma unroll
-                    for (int q = 0; q < R; ++q) a[i][cc][q] = src[q];
-                }
-            }
-        }
-    }
     __device__ __forceinline__ void butterflies(int i, int u, const float2 *tw, int stepR, int M) {
         if (u > 0) {
 #pragma unroll
@@ -387,43 +359,43 @@ __device__ void fft_pass_wg(float2 *buf, const float2 *tw, int N, const FFTPass 
 }
 
 // Last pass (M = 1, u = t) with its results stored straight to the grid: point u + l s of a
-// butterfly's columns, so neighbouring lanes store neighbouring points.
-template <int R, bool INV, class PC>
-__device__ __forceinline__ void fft_last_columns(const float2 *buf, const float2 *tw, int N, const FFTPass &pd,
-                                                 const GridRings &out, int tid) {
-    typedef PassRegs<R, INV, PC> Regs;
-    constexpr int CB = Regs::CB, SC = kFFTCols / PC::SUB;
-    const int nb = N / R, items = nb * Regs::NCG;
-    const FastDiv divM(1, 0u);
+// butterfly's column, so neighbouring lanes store neighbouring points.  Nothing is written to
+// LDS, so the items (one column each) run in a loop.  Even radices read their consecutive
+// inputs in pairs (16-byte aligned: rings have a multiple of 4 points).
+template <int R, bool INV>
+__device__ void fft_last_pass(const float2 *buf, const float2 *tw, int N, const GridRings &out, int tid) {
+    const int nb = N / R, items = nb * out.ncol;
+#pragma unroll 1
+    for (int it = tid; it < items; it += kFFTThreads) {
+        int c = 0;
 #pragma unroll
-    for (int sp = 0; sp < PC::SUB; ++sp) {
-        Regs x;
-        x.read_last(buf + sp * SC * N, N, tid);
+        for (int k = 1; k < kFFTCols; ++k) c += it >= k * nb ? 1 : 0;
+        const int u = it - c * nb;
+        const float2 *src = buf + c * N + R * u;
+        float2 a[R];
+        if constexpr (R % 2 == 0) {
 #pragma unroll
-        for (int i = 0; i < Regs::MAXI; ++i) {
-            const int it = tid + kFFTThreads * i;
-            if (it >= items) continue;
-            const PassItem<PC> p(it, nb, divM);
-            x.butterflies(i, p.u, tw, N / R, pd.M);
-#pragma unroll
-            for (int cc = 0; cc < CB; ++cc) {
-                const int c = sp * SC + p.cg * CB + cc;
-                if (c >= out.ncol) continue;
-                SHT_GLOBAL float *fn = out.fn + c * out.ld + p.u, *fs = out.fs + c * out.ld + p.u;
-#pragma unroll
-                for (int s = 0; s < R; ++s) {
-                    fn[(unsigned)(nb * s)] = x.a[i][cc][s].x;
-                    fs[(unsigned)(nb * s)] = x.a[i][cc][s].y;
-                }
+            for (int q = 0; q < R; q += 2) {
+                const float4 v = *reinterpret_cast<const float4 *>(src + q);
+                a[q] = make_float2(v.x, v.y);
+                a[q + 1] = make_float2(v.z, v.w);
             }
+        } else {
+#pragma unroll
+            for (int q = 0; q < R; ++q) a[q] = src[q];
+        }
+        if (u > 0) {
+#pragma unroll
+            for (int q = 1; q < R; ++q) a[q] = cmul(a[q], twid<INV>(tw, q * u));
+        }
+        bfly_any<R, INV>(a, tw, nb);
+        SHT_GLOBAL float *fn = out.fn + c * out.ld + u, *fs = out.fs + c * out.ld + u;
+#pragma unroll
+        for (int s = 0; s < R; ++s) {
+            fn[(unsigned)(nb * s)] = a[s].x;
+            fs[(unsigned)(nb * s)] = a[s].y;
         }
     }
-}
-
-template <int R, bool INV>
-__device__ void fft_last_pass(const float2 *buf, const float2 *tw, int N, const FFTPass &pd, const GridRings &out,
-                              int tid) {
-    pass_columns<R>(N / R, [&](auto pc) { fft_last_columns<R, INV, decltype(pc)>(buf, tw, N, pd, out, tid); });
 }
 
 // First pass (l = 1) of an odd prime radix r >= 11 as two small GEMMs on MFMA, in place.
@@ -637,15 +609,15 @@ __device__ __attribute__((always_inline)) void fft_run(const FFTPlanTables &P, c
         int t = tid;
         asm volatile("" : "+v"(t));
         switch (pd.R) {
-            case 16: fft_last_pass<16, INV>(buf, tw, N, pd, out, t); break;
-            case 8: fft_last_pass<8, INV>(buf, tw, N, pd, out, t); break;
-            case 2: fft_last_pass<2, INV>(buf, tw, N, pd, out, t); break;
-            case 3: fft_last_pass<3, INV>(buf, tw, N, pd, out, t); break;
-            case 4: fft_last_pass<4, INV>(buf, tw, N, pd, out, t); break;
-            case 5: fft_last_pass<5, INV>(buf, tw, N, pd, out, t); break;
-            case 7: fft_last_pass<7, INV>(buf, tw, N, pd, out, t); break;
-            case 11: fft_last_pass<11, INV>(buf, tw, N, pd, out, t); break;
-            default: fft_last_pass<13, INV>(buf, tw, N, pd, out, t); break;
+            case 16: fft_last_pass<16, INV>(buf, tw, N, out, t); break;
+            case 8: fft_last_pass<8, INV>(buf, tw, N, out, t); break;
+            case 2: fft_last_pass<2, INV>(buf, tw, N, out, t); break;
+            case 3: fft_last_pass<3, INV>(buf, tw, N, out, t); break;
+            case 4: fft_last_pass<4, INV>(buf, tw, N, out, t); break;
+            case 5: fft_last_pass<5, INV>(buf, tw, N, out, t); break;
+            case 7: fft_last_pass<7, INV>(buf, tw, N, out, t); break;
+            case 11: fft_last_pass<11, INV>(buf, tw, N, out, t); break;
+            default: fft_last_pass<13, INV>(buf, tw, N, out, t); break;
         }
     }
 }
@@ -681,11 +653,12 @@ struct FFTTile {
     int k0, ncol;
 };
 
-// Single-call launch orders, rings heaviest first.  Paired (synthesis, which reads the
-// Fourier rows): units (ring rank r, column-group pair p) go round-robin to the XCDs and
-// the two column groups of a unit, which share the 128-byte lines of the Fourier rows, run
-// back to back on the same XCD: block b -> XCD b % 8, slot s = b / 8, unit
-// (s / 2) * 8 + b % 8, column group 2 p + s % 2.  Otherwise (analysis): block b -> ring
+// Single-call launch orders, rings heaviest first.  Grouped: every column group of ring rank r
+// on XCD r % 8 (blocks go round-robin over the XCDs), so the ring's twiddles and tables are
+// fetched into one L2, and the two column groups that share the 128-byte lines of the Fourier
+// rows (64 bytes each) meet in it: T255 K=64 with buffers that are not cache-resident, the
+// analysis, which writes those rows, takes 34.1 us with its column groups spread over the
+// XCDs and 30.3 us grouped.  Otherwise (a tuning choice of the synthesis): block b -> ring
 // rank b / kgs, column group b % kgs.  Batch tiles carry the rank (m) and column group.
 // rings: the plan's ring records (single calls pass them in place of a tile list), followed by
 // copies of the first marked j < 0 up to a multiple of the XCD count: blocks past the last ring
@@ -701,9 +674,6 @@ __device__ inline void fft_tile(const SHT_GLOBAL FFTRing *rings, const Tile &T, 
     } else {
         const int b = blockIdx.x;
         if (paired) {
-            // every column group of ring rank r on XCD r % 8 (blocks go round-robin over the
-            // XCDs), ranks heaviest first on each: the ring's twiddles and tables are fetched
-            // into one L2, and the column groups sharing a line of Fourier rows meet there
             const int s = b / kXCDs;
             r = (s / kgs) * kXCDs + b % kXCDs;
             cg = s - (s / kgs) * kgs;
@@ -845,7 +815,7 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
         BATCH ? as_global(P.rings) : as_global(reinterpret_cast<const FFTRing *>(tiles));
     const FFTPlanTables tables{P.twiddle, P.passes, P.prime_tab};
     FFTTile G;
-    fft_tile<BATCH>(rings, T, K, false, G);
+    fft_tile<BATCH>(rings, T, K, true, G);
     const FFTRing &R = G.R;
     const int N = R.N, mt = R.mt, ncol = G.ncol;
     __builtin_assume(N >= 1 && N <= kFFTMaxRing);  // offsets within a ring fit scalar-base loads

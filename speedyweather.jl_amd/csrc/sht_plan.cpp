@@ -1292,7 +1292,7 @@ static StageLaunch plan_stage_launch(const sht_plan *plan, int stage, const Call
                 return {sht::fft_kernel(stage, false, c.accumulate != 0), dim3(fft_blocks(plan->g.n, K, c.paired != 0)),
                         (unsigned)plan->P.fft_smem, reinterpret_cast<const Tile *>(plan->P.rings)};
             // the FFT kernels of a single call take the ring records in place of a tile list
-            return {sht::fft_kernel(stage, false), dim3(fft_blocks(plan->g.n, K, false)), (unsigned)plan->P.fft_smem,
+            return {sht::fft_kernel(stage, false), dim3(fft_blocks(plan->g.n, K, true)), (unsigned)plan->P.fft_smem,
                     reinterpret_cast<const Tile *>(plan->P.rings)};
         }
         default:
