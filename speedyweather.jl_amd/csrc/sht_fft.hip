@@ -707,7 +707,7 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
     const Tile T = BATCH ? tiles[blockIdx.x] : Tile{0, 0, 0, 0};
     if (BATCH && T.m < 0) return;  // padding of the launch order
     const CallArgs C = BATCH ? calls[T.call] : single;
-    const DevPlan &P = plans[C.plan];
+    const DevPlan &P = plans[BATCH ? C.plan : 0];
     const int K = C.K;
     const SHT_GLOBAL FFTRing *rings =
         BATCH ? as_global(P.rings) : as_global(reinterpret_cast<const FFTRing *>(tiles));
@@ -809,7 +809,7 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
     const Tile T = BATCH ? tiles[blockIdx.x] : Tile{0, 0, 0, 0};
     if (BATCH && T.m < 0) return;  // padding of the launch order
     const CallArgs C = BATCH ? calls[T.call] : single;
-    const DevPlan &P = plans[C.plan];
+    const DevPlan &P = plans[BATCH ? C.plan : 0];
     const int K = C.K;
     const SHT_GLOBAL FFTRing *rings =
         BATCH ? as_global(P.rings) : as_global(reinterpret_cast<const FFTRing *>(tiles));

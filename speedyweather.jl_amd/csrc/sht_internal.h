@@ -79,6 +79,21 @@ struct Tile {
     int cg;
 };
 
+// A Legendre tile as the kernels read it: the tile and everything of its order that its loads
+// depend on, so that they follow after one level of scalar loads.  skip: padding of the launch
+// order (the other fields copy a real tile, so the workgroup may issue loads before it exits).
+struct LegTile {
+    Tile t;
+    int j0, J;         // first ring with the order and their count
+    int L;             // degrees of the order
+    int skip;
+    long long lm_off;  // packed offset of the order's column
+    long long off;     // the order's block in the stage's Λ arrays
+    long long soff;    // the order's row scales
+    long long pad;
+};
+static_assert(sizeof(LegTile) == 64, "LegTile layout");
+
 // A column of a merged Legendre column group: batch items on one plan (and, for the
 // synthesis, one unscale_coslat flag) share column groups of kColsComplex columns, so one
 // workgroup (order m, ring or degree block) reads Λ once for all of them.  Group q's columns
@@ -202,6 +217,7 @@ struct DevPlan {
     int lmax, mmax;   // 1-based
     int nharm;
     long long npoints;
+    int fb_a, fb_b;   // first Fourier-buffer row of ring j: j (fb_a j + fb_b)
     int kg;           // columns per FFT workgroup
     int fft_smem;     // dynamic LDS bytes of the FFT kernel
 
@@ -289,9 +305,9 @@ int static_scratch_setup(int device);
 
 // Kernel entry points.  Every stage kernel takes
 //   (const DevPlan *plans, CallArgs single, const CallArgs *calls, const Tile *tiles)
-// on a 1-D grid.  batch = false: the single call's arguments by value; the Legendre
-// kernels read their tile from tiles[blockIdx.x], the FFT kernels derive ring and column
-// group from blockIdx.x.  batch = true: tile, call and column group from tiles.
+// on a 1-D grid.  batch = false: the single call's arguments by value on plans[0]; the Legendre
+// kernels read their tile from the LegTile list passed as tiles (batches too), the FFT kernels
+// derive ring and column group from blockIdx.x.  batch = true: tile, call and column group from tiles.
 const void *legendre_kernel(int stage, int mode, bool batch);
 const void *legendre_mixed_kernel(int mode);  // single-call synthesis with CallArgs::mixed
 // accumulate: the single-call synthesis that adds into its output (pullbacks); batches

@@ -122,6 +122,23 @@ __device__ __forceinline__ const SHT_GLOBAL CallArgs *call_of(const CallArgs *ca
     return as_global(calls) + (call < 0 ? call0 : call);
 }
 
+// A tile record read field by field (structures do not copy through global pointers).
+__device__ __forceinline__ LegTile load_leg_tile(const Tile *tiles) {
+    const SHT_GLOBAL int *q = as_global(reinterpret_cast<const int *>(tiles)) + (size_t)blockIdx.x * (sizeof(LegTile) / 4);
+    const SHT_GLOBAL long long *w = reinterpret_cast<const SHT_GLOBAL long long *>(q);
+    LegTile r;
+    r.t = Tile{q[0], q[1], q[2], q[3]};
+    r.j0 = q[4];
+    r.J = q[5];
+    r.L = q[6];
+    r.skip = q[7];
+    r.lm_off = w[4];
+    r.off = w[5];
+    r.soff = w[6];
+    r.pad = 0;
+    return r;
+}
+
 // acc[t] += A_t (16 rows x 32 contraction, this lane's fragment of row tile t < TPW) x B
 // tile columns cb*16..cb*16+15 of parity p; each B fragment is read once for all TPW row
 // tiles.  FP32: af[t][8] holds the lane's A values of tile t for the 8 K-steps of 4.
@@ -207,9 +224,10 @@ __device__ inline void mma_chunk1(const unsigned char *sm, int buf, int p, int r
 // order of K within every chunk (sht_plan.cpp: syn_kpos).
 
 
-// Per-ring epilogue factors of ring rb < 64 of a synthesis block: 16 bytes in the padding of
+// Per-ring epilogue factor of ring rb < 64 of a synthesis block: 8 bytes in the padding of
 // staging row rb (parity 0, buffer 0; the FP32 row, or the lo row of the split modes), which
-// the staging and the products never touch: the Fourier row offset, then the row scale.
+// the staging and the products never touch: the row scale with 1 / cos(lat), then (MIXED)
+// without.
 // Degree factor of a fused Laplacian: lap 1: e_l = -l(l+1); lap 2: 1 / e_l, 0 at l = 0.
 __device__ __forceinline__ float lap_factor(int lap, int l) {
     const float e = -(float)l * (float)(l + 1);
@@ -234,27 +252,25 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
                                                                  const Tile *__restrict__ tiles) {
     // the wave index is uniform per wave: keep it (and all tile ownership) scalar
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const Tile T = tiles[blockIdx.x];
-    if (T.m < 0) return;  // padding of the launch order
+    const LegTile R = load_leg_tile(tiles);
+    const Tile &T = R.t;
     const SHT_GLOBAL ColRef *cmap = merged_columns<BATCH>(T, single);
     const int call0 = cmap ? column_ref(cmap, 0).call : T.call;
     const CallArgs C = BATCH ? calls[call0] : single;
-    const DevPlan &P = plans[C.plan];
+    const DevPlan &P = plans[BATCH ? C.plan : 0];
     const int m = T.m, cg = T.cg;
     const SHT_GLOBAL float2 *coeffs = as_global(static_cast<const float2 *>(C.in));
     const long long ld_spec = C.ld_in;
     SHT_GLOBAL float4 *fbuf = as_global(static_cast<float4 *>(C.fbuf));
     const int K = C.K, unscale = C.unscale;
-    const int n = P.n;
-    const int j0 = as_global(P.j0)[m];
-    const int J = n - j0;
-    const int L = P.lmax - m;
+    const int fb_a = P.fb_a, fb_b = P.fb_b;
+    const int j0 = R.j0, J = R.J, L = R.L;
     const int Le = (L + 1) >> 1;
     const int nch = (Le + kChunk - 1) / kChunk;
     const int Jt = (J + 15) >> 4;
     const int tile = T.blk * 4 + w;
     const bool active = tile < Jt;
-    const long long off = as_global(P.lm_off)[m];
+    const long long off = R.lm_off;
     const int kbase = cg * kColsComplex;
     const int row = lane & 15, grp = lane >> 4;
     // staging role
@@ -288,7 +304,7 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
         V8of<MODE> ap[2][3];  // [parity][part]
     };
     const int ltile = active ? tile : Jt - 1;
-    const long long so = as_global(P.syn_off)[m];
+    const long long so = R.off;
     const SHT_GLOBAL float *Af[2];
     const SHT_GLOBAL V8of<MODE> *Ap[2][3];
 #pragma unroll
@@ -350,27 +366,25 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
         }
     };
 
-    // straight-line loop body (a conditional second step would make the waits at the loop
-    // head cover every outstanding load)
-    // Per-ring epilogue factors of this block's 64 rings (Fourier row offset, FP16 row scale,
-    // 1 / cos(lat)), loaded before the first chunk and kept in LDS until the epilogue.
-    static_assert(kRowF - kChunk >= 4 && kRowH - kChunk >= 8, "16 bytes of row padding");
-    long long e_row = 0;
-    float e_sc = 1.f, e_ci = 1.f;
-    if (w == 0) {
-        const int r = min(64 * T.blk + lane, J - 1);  // ring j0 + r
-        e_row = as_global(P.fboff)[j0 + r] + m;
-        if constexpr (MODE == kFP16x3) e_sc = as_global(P.syn_sinv)[as_global(P.syn_soff)[m] + r];
-        if (unscale) e_ci = as_global(P.coslat_inv)[j0 + r];
-    }
+    // Per-ring epilogue factors of this block's 64 rings (FP16 row scale, 1 / cos(lat)), loaded
+    // behind the first chunk and kept in LDS until the epilogue.
+    static_assert(kRowF - kChunk >= 2 && kRowH - kChunk >= 4, "8 bytes of row padding");
     Ops S0, S1;
     load(S0, 0);
+    float e_sc = 1.f, e_ci = 1.f;
+    {
+        const int r = min(64 * T.blk + lane, J - 1);  // ring j0 + r
+        if constexpr (MODE == kFP16x3) e_sc = as_global(P.syn_sinv)[R.soff + r];
+        if (unscale) e_ci = as_global(P.coslat_inv)[j0 + r];
+    }
+    if (R.skip) return;  // padding of the launch order
     if (w == 0) {
         unsigned char *slot = ep_slot<MODE>(sm, lane);
-        *reinterpret_cast<long long *>(slot) = e_row;
-        *reinterpret_cast<float *>(slot + 8) = e_sc * e_ci;
-        if constexpr (MIXED) *reinterpret_cast<float *>(slot + 12) = e_sc;
+        *reinterpret_cast<float *>(slot) = e_sc * e_ci;
+        if constexpr (MIXED) *reinterpret_cast<float *>(slot + 4) = e_sc;
     }
+    // straight-line loop body (a conditional second step would make the waits at the loop
+    // head cover every outstanding load)
     int c = 0;
     for (; c + 1 < nch; c += 2) {
         step(S0, S1, c);
@@ -401,14 +415,14 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
             const int j = j0 + 16 * tile + r;
             const int rb = 16 * w + r;  // ring within the block
             const unsigned char *slot = ep_slot<MODE>(sm, rb);
-            const float sc = *reinterpret_cast<const float *>(slot + (MIXED && k >= unscale ? 12 : 8));
+            const float sc = *reinterpret_cast<const float *>(slot + (MIXED && k >= unscale ? 4 : 0));
             const float e = acc[0][cb][i] * sc, o = acc[1][cb][i] * sc;
             const float nv = e + o, sv = e - o;
             const float n_other = lane_xor1(nv);
             const float s_other = lane_xor1(sv);
-            if (j < n && kin) {
-                SHT_GLOBAL float2 *dst = reinterpret_cast<SHT_GLOBAL float2 *>(
-                    fb + *reinterpret_cast<const long long *>(slot) * (long long)Kk + k);
+            if (j < j0 + J && kin) {
+                SHT_GLOBAL float2 *dst =
+                    reinterpret_cast<SHT_GLOBAL float2 *>(fb + (long long)(j * (fb_a * j + fb_b) + m) * Kk + k);
                 if (reim == 0) {
                     gstore(dst, make_float2(nv, n_other));
                 } else {
@@ -438,27 +452,25 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 3) void legendre_analysi
     constexpr int kAnaTiles = DPW / 32;  // degree tiles per parity per workgroup
     // the wave index is uniform per wave: keep it (and all tile ownership) scalar
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const Tile T = tiles[blockIdx.x];
-    if (T.m < 0) return;  // padding of the launch order
+    const LegTile R = load_leg_tile(tiles);
+    const Tile &T = R.t;
     const SHT_GLOBAL ColRef *cmap = merged_columns<BATCH>(T, single);
     const int call0 = cmap ? column_ref(cmap, 0).call : T.call;
     const CallArgs C = BATCH ? calls[call0] : single;
-    const DevPlan &P = plans[C.plan];
+    const DevPlan &P = plans[BATCH ? C.plan : 0];
     const int m = T.m, cg = T.cg;
     const SHT_GLOBAL float4 *fbuf = as_global(static_cast<const float4 *>(C.fbuf));
     SHT_GLOBAL float2 *coeffs = as_global(static_cast<float2 *>(C.out));
     const long long ld_spec = C.ld_out;
     const int K = C.K;
-    const int n = P.n;
-    const int j0 = as_global(P.j0)[m];
-    const int J = n - j0;
-    const int L = P.lmax - m;
+    const int fb_a = P.fb_a, fb_b = P.fb_b;
+    const int j0 = R.j0, J = R.J, L = R.L, n = j0 + J;
     const int NG = (L + DPW - 1) / DPW;
     const int nt = kAnaTiles * NG;  // degree tiles per parity in the table
     const int JC = (J + kChunk - 1) / kChunk;
     const int p = w & 1;
     const int lt0 = kAnaTiles * T.blk + TPW * (w >> 1);  // first degree tile of this wave
-    const long long off = as_global(P.lm_off)[m];
+    const long long off = R.lm_off;
     const int kbase = cg * kColsComplex;
     const int row = lane & 15, grp = lane >> 4;
     const int kk = stage_column<MODE>(tid), g = tid & 7;
@@ -483,29 +495,18 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 3) void legendre_analysi
     for (int t = 0; t < TPW; ++t)
 #pragma unroll
         for (int cb = 0; cb < 4; ++cb) acc[t][cb] = f4{0.f, 0.f, 0.f, 0.f};
-    // FP16 row scales of this lane's output rows, loaded now for the epilogue
-    float rs[TPW][4];
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            rs[t][i] = MODE == kFP16x3 ? as_global(P.ana_sinv)[as_global(P.ana_soff)[m] + (p * nt + lt0 + t) * 16 + 4 * grp + i]
-                                       : 1.f;
-
     // Operands of one chunk: 4 rings of one column (staging role) and this wave's Λ
     // fragments.  Two sets alternate (no register copies between chunks); the next chunk's
     // set is loaded while the current chunk's products run.  All loads are unconditional
     // (rings past n re-read ring n - 1, absent columns column 0, the step after the last
     // chunk the last chunk again; the staging zeroes what is not data), so each wait covers
-    // exactly the loads it needs.  A set also carries the Fourier row offsets of the chunk
-    // after its own, loaded ahead of its rows, so no Fourier load waits for the offset table.
+    // exactly the loads it needs.
     struct Ops {
         float4 v[4];
         float af[TPW][8];
         V8of<MODE> ap[TPW][3];  // [tile][part]
-        int fo[4];  // first Fourier rows of the following chunk's rings (< 2^31 rows)
     };
-    const long long ao = as_global(P.ana_off)[m];
+    const long long ao = R.off;
     const SHT_GLOBAL float *Af[TPW];
     const SHT_GLOBAL V8of<MODE> *Ap[TPW][3];
 #pragma unroll
@@ -519,17 +520,13 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 3) void legendre_analysi
                            static_cast<const u16 *>(lam_part<MODE>(P.ana_hi, P.ana_mid, P.ana_lo, q)) + ao)) +
                        fi;
     }
-    auto load_offsets = [&](int (&fo)[4], int c) {
+    auto load = [&](Ops &S, int c) {
         c = min(c, JC - 1);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) fo[i] = (int)as_global(P.fboff)[min(j0 + kChunk * c + 4 * g + i, n - 1)];
-    };
-    // chunk c into S, given the ring offsets fo of chunk c
-    auto load = [&](Ops &S, int c, const int (&fo)[4]) {
-        c = min(c, JC - 1);
-        load_offsets(S.fo, c + 1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) S.v[i] = gload(sfb + (long long)(fo[i] + m) * sK + kgl);
+        for (int i = 0; i < 4; ++i) {
+            const int j = min(j0 + kChunk * c + 4 * g + i, n - 1);
+            S.v[i] = gload(sfb + (long long)(j * (fb_a * j + fb_b) + m) * sK + kgl);
+        }
 #pragma unroll
         for (int t = 0; t < TPW; ++t) {
             if constexpr (MODE == kFP32) {
@@ -559,16 +556,22 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 3) void legendre_analysi
             im[i] = ok[i] ? cur.v[i].w : 0.f;
         }
         stage4<MODE>(sm, buf, 1, kk, g, re, im);
-        load(nxt, c + 1, cur.fo);
+        load(nxt, c + 1);
         __syncthreads();
         mma_chunk<MODE, 4, TPW>(sm, buf, p, row, grp, cur.af, cur.ap, acc);
     };
 
-    if (JC > 0) {  // no rings for this order: the coefficients are zero
-        Ops S0, S1;
-        int fo0[4];
-        load_offsets(fo0, 0);
-        load(S0, 0, fo0);
+    Ops S0, S1;
+    if (JC > 0) load(S0, 0);  // no rings for this order: the coefficients are zero
+    // FP16 row scales of this lane's output rows, loaded behind the first chunk for the epilogue
+    float rs[TPW][4];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            rs[t][i] = MODE == kFP16x3 ? as_global(P.ana_sinv)[R.soff + (p * nt + lt0 + t) * 16 + 4 * grp + i] : 1.f;
+    if (R.skip) return;  // padding of the launch order
+    if (JC > 0) {
         int c = 0;
         for (; c + 1 < JC; c += 2) {  // straight-line body, as in the synthesis
             step(S0, S1, c);

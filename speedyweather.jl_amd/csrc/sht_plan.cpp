@@ -364,6 +364,7 @@ struct sht_plan {
     // host copies for batches: Legendre tiles (heavy first) with their costs, FFT ring order
     // and cost per policy
     std::vector<Tile> h_syn, h_ana;
+    std::vector<long long> h_off[2], h_soff[2];  // Λ and scale offsets per order (synthesis, analysis)
     std::vector<double> h_syn_cost, h_ana_cost, h_ring_cost_v[kPolicies];
     std::vector<int> h_ring_order_v[kPolicies];
     // Scratch per stream: the Fourier buffer (fb_bytes), or on matrix plans also the dense
@@ -439,6 +440,27 @@ void free_plan(sht_plan *p) {
     for (void *a : p->allocs) (void)hipFree(a);
     for (auto &sb : p->scratch) (void)hipFree(sb.second);
     delete p;
+}
+
+// Uploads a Legendre launch order as the records the kernels read (LegTile); plan_of gives a
+// tile's plan.  Padding copies the first real tile.
+template <class F>
+int upload_leg_tiles(std::vector<void *> &allocs, const std::vector<Tile> &order, int stage, F plan_of, const Tile **out) {
+    std::vector<sht::LegTile> rec(order.size());
+    const int ana = stage == sht::kLegendreAnalysis ? 1 : 0;
+    size_t first = 0;
+    while (first < order.size() && order[first].m < 0) ++first;
+    for (size_t i = 0; i < order.size(); ++i) {
+        const Tile &t = order[i].m < 0 ? order[first] : order[i];
+        const sht_plan *pl = plan_of(t);
+        const Geometry &g = pl->g;
+        rec[i] = sht::LegTile{t, g.j0[t.m], g.n - g.j0[t.m], g.lmax - t.m, order[i].m < 0 ? 1 : 0,
+                              g.lm_off[t.m], pl->h_off[ana][t.m], pl->h_soff[ana][t.m], 0};
+    }
+    const sht::LegTile *p = nullptr;
+    const int rc = dev_upload(allocs, rec, &p);
+    *out = reinterpret_cast<const Tile *>(p);
+    return rc;
 }
 
 // The scratch of `stream` on this plan (allocated on the stream's first call), or null
@@ -859,6 +881,10 @@ int build_plan(sht_plan *pl) {
     sort_tiles(ana_t, ana_c);
     pl->h_syn = syn_t;
     pl->h_ana = ana_t;
+    pl->h_off[0] = syn_off;
+    pl->h_off[1] = ana_off;
+    pl->h_soff[0] = syn_soff;
+    pl->h_soff[1] = ana_soff;
     pl->h_syn_cost = syn_c;
     pl->h_ana_cost = ana_c;
 
@@ -884,6 +910,10 @@ int build_plan(sht_plan *pl) {
 
     // --------------------------------------------------------------- upload
     std::vector<float> coslat_f(coslat_inv.begin(), coslat_inv.end());
+    P.fb_a = d.grid == SHT_GRID_OCTAHEDRAL_GAUSSIAN ? 1 : 0;
+    P.fb_b = P.fb_a ? 10 : 2 * n + 1;
+    for (int j = 0; j < n; ++j)
+        if (g.fboff[j] != (long long)j * (P.fb_a * j + P.fb_b)) return fail(SHT_ERR_UNSUPPORTED, "Fourier row layout");
     P.n = n; P.lmax = lmax; P.mmax = mmax; P.nharm = g.nharm; P.npoints = g.npoints;
     if ((rc = dev_upload(A, g.nlon, &P.nlon))) return rc;
     if ((rc = dev_upload(A, g.mt, &P.mt))) return rc;
@@ -1005,8 +1035,8 @@ int build_plan(sht_plan *pl) {
                     }
                 }
                 const Tile *ds = nullptr, *da = nullptr;
-                if ((rc = dev_upload(A, so, &ds))) return rc;
-                if ((rc = dev_upload(A, ao, &da))) return rc;
+                if ((rc = upload_leg_tiles(A, so, sht::kLegendreSynthesis, [&](const Tile &) { return pl; }, &ds))) return rc;
+                if ((rc = upload_leg_tiles(A, ao, sht::kLegendreAnalysis, [&](const Tile &) { return pl; }, &da))) return rc;
                 pl->syn_tiles[variant].push_back(ds);
                 pl->ana_tiles[variant].push_back(da);
                 pl->nsyn[variant].push_back((int)so.size());
@@ -2163,7 +2193,18 @@ int build_batch(sht_batch *b, const sht_batch_item *items, int n, int flags) {
         // heaviest units first across all items, spread over the XCDs
         const std::vector<Tile> order = st_units[st].empty() ? std::vector<Tile>() : xcd_order(st_units[st]);
         b->ntiles[st] = (int)order.size();
-        if (!order.empty() && (rc = dev_upload(b->allocs, order, &b->tiles[st]))) return rc;
+        if (order.empty()) continue;
+        if (st == sht::kLegendreSynthesis || st == sht::kLegendreAnalysis)
+            rc = upload_leg_tiles(
+                b->allocs, order, st,
+                [&](const Tile &t) {
+                    const int call = t.call >= 0 ? t.call : colmap[(size_t)(-1 - t.call) * sht::kColsComplex].call;
+                    return plans[calls[call].plan];
+                },
+                &b->tiles[st]);
+        else
+            rc = dev_upload(b->allocs, order, &b->tiles[st]);
+        if (rc) return rc;
     }
     if (b->fft_smem > 65536) {
         for (int st : {sht::kFFTSynthesis, sht::kFFTAnalysis})
