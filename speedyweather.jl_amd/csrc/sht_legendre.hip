@@ -409,26 +409,26 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
             Kk = ck->K;
             fb = as_global(static_cast<float4 *>(ck->fbuf));
         }
+        // rows in pairs: the lanes of a column exchange halves, the even one stores row i, the
+        // odd one row i + 1, 16 bytes each
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 4; i += 2) {
             const int r = 4 * grp + i;
-            const int j = j0 + 16 * tile + r;
-            const int rb = 16 * w + r;  // ring within the block
-            const unsigned char *slot = ep_slot<MODE>(sm, rb);
-            const float sc = *reinterpret_cast<const float *>(slot + (MIXED && k >= unscale ? 4 : 0));
-            const float e = acc[0][cb][i] * sc, o = acc[1][cb][i] * sc;
-            const float nv = e + o, sv = e - o;
-            const float n_other = lane_xor1(nv);
-            const float s_other = lane_xor1(sv);
-            if (j < j0 + J && kin) {
-                SHT_GLOBAL float2 *dst =
-                    reinterpret_cast<SHT_GLOBAL float2 *>(fb + (long long)(j * (fb_a * j + fb_b) + m) * Kk + k);
-                if (reim == 0) {
-                    gstore(dst, make_float2(nv, n_other));
-                } else {
-                    gstore(dst + 1, make_float2(s_other, sv));
-                }
+            float nv[2], sv[2], n_other[2], s_other[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const unsigned char *slot = ep_slot<MODE>(sm, 16 * w + r + h);  // ring within the block
+                const float sc = *reinterpret_cast<const float *>(slot + (MIXED && k >= unscale ? 4 : 0));
+                const float e = acc[0][cb][i + h] * sc, o = acc[1][cb][i + h] * sc;
+                nv[h] = e + o;
+                sv[h] = e - o;
+                n_other[h] = lane_xor1(nv[h]);
+                s_other[h] = lane_xor1(sv[h]);
             }
+            const int j = j0 + 16 * tile + r + reim;
+            const float4 v = reim == 0 ? make_float4(nv[0], n_other[0], sv[0], s_other[0])
+                                       : make_float4(n_other[1], nv[1], s_other[1], sv[1]);
+            if (j < j0 + J && kin) gstore(fb + (long long)(j * (fb_a * j + fb_b) + m) * Kk + k, v);
         }
     }
 }
