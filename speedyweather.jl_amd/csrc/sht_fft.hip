@@ -206,7 +206,7 @@ __device__ inline void bfly_any(float2 *a, const float2 *tw, int stepR) {
         bfly_odd<R, INV>(a, tw, stepR);
 }
 
-// A pass of radix R over all columns of N <= kFFTMaxRing points, run by the workgroup.
+// A pass of radix R over all columns of N <= MAXN points, run by the workgroup.
 // Work item = (column group of CB columns, butterfly t); items go to threads in order, so
 // neighbouring lanes take neighbouring butterflies of one column group.  The index
 // arithmetic and the twiddles of a butterfly serve all CB columns of its item.  Every
@@ -219,31 +219,28 @@ __device__ inline void bfly_any(float2 *a, const float2 *tw, int stepR) {
 // analysis; T127 K=32: 9.2 -> 8.8, 9.4 -> 9.2).
 // Radices 11 and 13 (one column per item) run as two sub-passes of two columns each where the
 // items of four columns exceed the threads.
-template <int R, int CBv, int SUBv = 1>
+template <int R, int MAXN, int CBv, int SUBv = 1>
 struct PassCols {
     static constexpr int CB = CBv;                   // columns per work item
     static constexpr int SUB = SUBv;                 // column sub-passes
     static constexpr int NCG = kFFTCols / CB / SUB;  // column groups per sub-pass
-    static constexpr int kMaxB = kFFTMaxRing / R;    // butterflies per column
+    static constexpr int kMaxB = MAXN / R;           // butterflies per column
     // the largest butterfly count this choice serves (pass_columns)
     static constexpr int kMaxNb = CB == 1 && SUB == 1 ? 64 : kMaxB;
     static constexpr int MAXI = ((kMaxNb < kMaxB ? kMaxNb : kMaxB) * NCG + kFFTThreads - 1) / kFFTThreads;
 };
 // Calls f with the column choice for nb butterflies per column.
-template <int R, class F>
+template <int R, int MAXN, class F>
 __device__ __forceinline__ void pass_columns(int nb, F &&f) {
-    if constexpr (R == 16) {  // nb <= 64
-        f(PassCols<R, 1>{});
-    } else if constexpr (R > 8) {
-        if (nb <= 64)
-            f(PassCols<R, 1>{});
-        else
-            f(PassCols<R, 1, 2>{});
+    if constexpr (MAXN / R <= 64) {
+        f(PassCols<R, MAXN, 1>{});
     } else {
         if (nb <= 64)
-            f(PassCols<R, 1>{});
+            f(PassCols<R, MAXN, 1>{});
+        else if constexpr (R > 8)
+            f(PassCols<R, MAXN, 1, 2>{});
         else
-            f(PassCols<R, 2>{});
+            f(PassCols<R, MAXN, 2>{});
     }
 }
 
@@ -257,8 +254,9 @@ struct GridRings {
 
 // Twiddles of a ring on their way to LDS: loaded together with the ring's data (one memory
 // latency for both), stored after every load of the thread is in flight.
+template <int MAXN>
 struct Twiddles {
-    static constexpr int U = (kFFTMaxRing + kFFTThreads - 1) / kFFTThreads;
+    static constexpr int U = MAXN / kFFTThreads;
     float2 v[U];
     __device__ __forceinline__ void load(const float *twiddle, long long tw_off, int N, int tid) {
         const SHT_GLOBAL float2 *g = as_global(reinterpret_cast<const float2 *>(twiddle)) + tw_off;
@@ -348,9 +346,9 @@ __device__ __forceinline__ void fft_subpass_wg(float2 *buf, const float2 *tw, in
     __syncthreads();
 }
 
-template <int R, bool INV>
+template <int R, bool INV, int MAXN>
 __device__ void fft_pass_wg(float2 *buf, const float2 *tw, int N, const FFTPass &pd, int tid) {
-    pass_columns<R>(N / R, [&](auto pc) {
+    pass_columns<R, MAXN>(N / R, [&](auto pc) {
         typedef decltype(pc) PC;
 #pragma unroll
         for (int sp = 0; sp < PC::SUB; ++sp)
@@ -414,7 +412,7 @@ __device__ void fft_last_pass(const float2 *buf, const float2 *tw, int N, const 
 // smallest first, so the pass keeps FP32-level accuracy in every precision mode.
 //
 // Column tiles go to the waves in rounds of four; with fewer column tiles left, the waves of
-// one column tile split its row tiles (at most kPrimeRowTiles per wave: rings of N = 4p
+// one column tile split its row tiles (at most prime_row_tiles(MAXN) per wave: rings of N = 4p
 // points have M = N / r >= 4, see sht_plan.cpp: factorize).  All row tiles of a round's
 // column tiles are computed before the workgroup synchronises and any output is written
 // (a butterfly's outputs overwrite its inputs, which the other row tiles still read).
@@ -454,13 +452,13 @@ __device__ inline f4 mma_bf16x3(const b8 &ah, const b8 &am, const b8 &al, const 
     return Split<kBF16x3>::mma(ah, bh, c);
 }
 
-template <bool INV>
+template <bool INV, int MAXN>
 __device__ void fft_pass_mfma_first(float2 *buf, const SHT_GLOBAL b8 *tab, int N, const FFTPass &pd, int ncol,
                                     int tmax, int tid) {
     const int r = pd.R, M = pd.M;
     const int h = (r - 1) >> 1;
     const int nseq = ncol * M;  // butterflies over all columns
-    constexpr int NW = kFFTThreads / 64;
+    constexpr int NW = kFFTThreads / 64, kRows = prime_row_tiles(MAXN);
     // the wave index is uniform per wave: keep it (and all tile ownership) scalar
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row = lane & 15, grp = lane >> 4, ri = row & 1;
@@ -474,10 +472,10 @@ __device__ void fft_pass_mfma_first(float2 *buf, const SHT_GLOBAL b8 *tab, int N
         const int nc = min(NW, Nt - n0);   // column tiles this round
         const int G = NW / nc;             // waves per column tile
         const int nt = n0 + wave % nc, r0 = wave / nc;
-        const int nrt = wave < nc * G ? min((Mt - r0 + G - 1) / G, kPrimeRowTiles) : 0;  // uniform per wave
-        f4 t1[kPrimeRowTiles], t2[kPrimeRowTiles];
+        const int nrt = wave < nc * G ? min((Mt - r0 + G - 1) / G, kRows) : 0;  // uniform per wave
+        f4 t1[kRows], t2[kRows];
 #pragma unroll
-        for (int i = 0; i < kPrimeRowTiles; ++i) t1[i] = t2[i] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < kRows; ++i) t1[i] = t2[i] = f4{0.f, 0.f, 0.f, 0.f};
         int ob = -1;
         float2 z0 = make_float2(0.f, 0.f);
         if (nrt > 0) {
@@ -505,7 +503,7 @@ __device__ void fft_pass_mfma_first(float2 *buf, const SHT_GLOBAL b8 *tab, int N
                 split3_bf16(xs, sh, sm, sl);
                 split3_bf16(xd, dh, dm, dl);
 #pragma unroll
-                for (int i = 0; i < kPrimeRowTiles; ++i) {
+                for (int i = 0; i < kRows; ++i) {
                     if (i >= nrt) break;  // uniform per wave
                     const SHT_GLOBAL b8 *a = tab + ((r0 + i * G) * KC + kc) * 384 + lane;
                     const b8 ch = a[0], cm = a[64], cl = a[128];
@@ -517,7 +515,7 @@ __device__ void fft_pass_mfma_first(float2 *buf, const SHT_GLOBAL b8 *tab, int N
         }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < kPrimeRowTiles; ++i) {
+        for (int i = 0; i < kRows; ++i) {
             if (i >= nrt) break;  // uniform per wave
             const int mt = r0 + i * G;
 #pragma unroll
@@ -565,7 +563,7 @@ struct FFTPlanTables {
     const unsigned short *prime_tab;
 };
 
-template <bool INV, bool LAST>
+template <bool INV, bool LAST, int MAXN>
 __device__ __attribute__((always_inline)) void fft_run(const FFTPlanTables &P, const FFTRing &R, float2 *buf,
                                                         const float2 *tw, int N, int mt, int ncol, FFTPass pd,
                                                         const GridRings &out, int tid) {
@@ -584,7 +582,7 @@ __device__ __attribute__((always_inline)) void fft_run(const FFTPlanTables &P, c
         const int tmax = INV ? min(h, (mt + p0.M - 1) / p0.M) : h;
         int t = tid;
         asm volatile("" : "+v"(t));
-        fft_pass_mfma_first<INV>(buf, tab, N, p0, ncol, max(tmax, 1), t);
+        fft_pass_mfma_first<INV, MAXN>(buf, tab, N, p0, ncol, max(tmax, 1), t);
         f = 1;
     }
     for (int g = f; g < nf - (LAST ? 1 : 0); ++g) {
@@ -593,15 +591,15 @@ __device__ __attribute__((always_inline)) void fft_run(const FFTPlanTables &P, c
         int t = tid;  // keeps every pass's index arithmetic inside the loop (hoisted, it spills)
         asm volatile("" : "+v"(t));
         switch (pd.R) {
-            case 16: fft_pass_wg<16, INV>(buf, tw, N, pd, t); break;
-            case 8: fft_pass_wg<8, INV>(buf, tw, N, pd, t); break;
-            case 2: fft_pass_wg<2, INV>(buf, tw, N, pd, t); break;
-            case 3: fft_pass_wg<3, INV>(buf, tw, N, pd, t); break;
-            case 4: fft_pass_wg<4, INV>(buf, tw, N, pd, t); break;
-            case 5: fft_pass_wg<5, INV>(buf, tw, N, pd, t); break;
-            case 7: fft_pass_wg<7, INV>(buf, tw, N, pd, t); break;
-            case 11: fft_pass_wg<11, INV>(buf, tw, N, pd, t); break;
-            default: fft_pass_wg<13, INV>(buf, tw, N, pd, t); break;  // the plan admits no other radix
+            case 16: fft_pass_wg<16, INV, MAXN>(buf, tw, N, pd, t); break;
+            case 8: fft_pass_wg<8, INV, MAXN>(buf, tw, N, pd, t); break;
+            case 2: fft_pass_wg<2, INV, MAXN>(buf, tw, N, pd, t); break;
+            case 3: fft_pass_wg<3, INV, MAXN>(buf, tw, N, pd, t); break;
+            case 4: fft_pass_wg<4, INV, MAXN>(buf, tw, N, pd, t); break;
+            case 5: fft_pass_wg<5, INV, MAXN>(buf, tw, N, pd, t); break;
+            case 7: fft_pass_wg<7, INV, MAXN>(buf, tw, N, pd, t); break;
+            case 11: fft_pass_wg<11, INV, MAXN>(buf, tw, N, pd, t); break;
+            default: fft_pass_wg<13, INV, MAXN>(buf, tw, N, pd, t); break;  // the plan admits no other radix
         }
         pd = nx;
     }
@@ -689,18 +687,24 @@ __device__ inline void fft_tile(const SHT_GLOBAL FFTRing *rings, const Tile &T, 
 
 // Fourier rows are read and written with thread -> (order mm = tid/4 + 64 u, column tid%4).
 constexpr int kFFTRowsPerPass = kFFTThreads / kFFTCols;
-constexpr int kFFTRowPasses = (kFFTMaxRing / 2 + kFFTRowsPerPass) / kFFTRowsPerPass;
+constexpr int fft_row_passes(int max_ring) { return (max_ring / 2 + kFFTRowsPerPass) / kFFTRowsPerPass; }
+// Workgroups (4 waves) per CU that a class is compiled for.  The passes wait on LDS more than they
+// compute, so what bounds short rings is workgroups in flight, and registers (512 per SIMD lane)
+// limit these before LDS does: 80 registers for rings of up to 512 points against 96 of the general
+// kernel, with no loads past the ring's length.  T127 K=392 synthesis + analysis 46.7 + 49.2 ->
+// 40.7 + 42.3 us, K=32 9.0 + 9.1 -> 8.6 + 8.4, T31 K=8 4.8 + 4.9 -> 4.2 + 4.2; a 7th workgroup
+// spills (T127 K=392 49.4 + 41.3).
+constexpr int fft_waves(int max_ring) { return max_ring <= 512 ? 6 : 5; }
 
 // spectral -> grid, Fourier stage (fourier.jl:215-250): per ring, brfft of g_N and g_S as
 // one complex inverse FFT of Z = g_N + i g_S (Hermitian-extended; Im of the DC and
 // Nyquist bins ignored as FFTW's c2r does; orders above mt are zero).  ACC: the pullback
 // that adds into the caller's grid (its own instantiation, so the plain transform keeps
 // its registers).
-template <bool BATCH, bool ACC = false>
-__global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const DevPlan *__restrict__ plans,
-                                                                    CallArgs single,
-                                                                    const CallArgs *__restrict__ calls,
-                                                                    const Tile *__restrict__ tiles) {
+template <int MAXN, bool BATCH, bool ACC = false>
+__global__ __launch_bounds__(kFFTThreads, fft_waves(MAXN))
+void fft_synthesis_kernel(const DevPlan *__restrict__ plans, CallArgs single, const CallArgs *__restrict__ calls,
+                          const Tile *__restrict__ tiles) {
     extern __shared__ float4 smem4[];
     float2 *smem = reinterpret_cast<float2 *>(smem4);
     const int tid = threadIdx.x;
@@ -716,20 +720,21 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
     fft_tile<BATCH>(rings, T, K, C.paired != 0, G);
     const FFTRing &R = G.R;
     const int N = R.N, mt = R.mt, ncol = G.ncol;
-    __builtin_assume(N >= 1 && N <= kFFTMaxRing);  // offsets within a ring fit scalar-base loads
+    __builtin_assume(N >= 1 && N <= MAXN);  // offsets within a ring fit scalar-base loads
     float2 *tw = smem;
     float2 *b0 = smem + N;
     const FFTPass pass0 = load_pass(as_global(tables.passes) + R.passes + (R.prime ? min(1, R.nf - 1) : 0));
-    Twiddles twr;
+    Twiddles<MAXN> twr;
     twr.load(tables.twiddle, R.tw_off, N, tid);
+    constexpr int kRowPasses = fft_row_passes(MAXN);
     {
         const SHT_GLOBAL float4 *fb =
             as_global(static_cast<const float4 *>(C.fbuf)) + R.fboff * (long long)K + G.k0;
         const int half = N / 2;
         const int col = tid % kFFTCols, m0 = tid / kFFTCols;
-        float4 v[kFFTRowPasses];
+        float4 v[kRowPasses];
 #pragma unroll
-        for (int u = 0; u < kFFTRowPasses; ++u) {
+        for (int u = 0; u < kRowPasses; ++u) {
             const int mm = m0 + kFFTRowsPerPass * u;
             v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (col < ncol && mm <= mt) v[u] = gload(fb + (unsigned)(mm * K + col));
@@ -740,7 +745,7 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
         if (C.adj) {  // adjoint of the analysis (grid2spec pullback): rows times ΔΩ_j / s_m
             const float wj = as_global(P.domega)[R.j];
 #pragma unroll
-            for (int u = 0; u < kFFTRowPasses; ++u) {
+            for (int u = 0; u < kRowPasses; ++u) {
                 const int mm = m0 + kFFTRowsPerPass * u;
                 const float sw = mm == 0 || 2 * mm == N ? wj : 0.5f * wj;
                 v[u] = make_float4(v[u].x * sw, v[u].y * sw, v[u].z * sw, v[u].w * sw);
@@ -748,7 +753,7 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
         }
         float2 *z = b0 + col * N;
 #pragma unroll
-        for (int u = 0; u < kFFTRowPasses; ++u) {
+        for (int u = 0; u < kRowPasses; ++u) {
             const int mm = m0 + kFFTRowsPerPass * u;
             if (col >= ncol || mm > half) continue;
             const float4 w = v[u];
@@ -765,11 +770,11 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
     __syncthreads();
     SHT_GLOBAL float *field = as_global(static_cast<float *>(C.out)) + (long long)G.k0 * C.ld_out;
     const GridRings out{field + R.ring_n, field + R.ring_s, C.ld_out, ncol};
-    fft_run<true, !ACC>(tables, R, b0, tw, N, mt, ncol, pass0, out, tid);
+    fft_run<true, !ACC, MAXN>(tables, R, b0, tw, N, mt, ncol, pass0, out, tid);
     if constexpr (ACC) {
         // pullback: add into the caller's cotangent; a column's old values are all read before
         // its first store, so the reads are in flight together
-        constexpr int U = (kFFTMaxRing + kFFTThreads - 1) / kFFTThreads;
+        constexpr int U = MAXN / kFFTThreads;
 #pragma unroll
         for (int c = 0; c < kFFTCols; ++c) {
             if (c >= ncol) break;  // uniform
@@ -798,8 +803,9 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_synthesis_kernel(const Dev
 // grid -> spectral, Fourier stage (fourier.jl:129-166): per ring, rfft of the northern and
 // southern ring as one complex FFT of z = f_N + i f_S, separated by symmetry into f_N, f_S
 // and stored as (f_N + f_S, f_N - f_S) for orders 0..mt.
-template <bool BATCH>
-__global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevPlan *__restrict__ plans,
+template <int MAXN, bool BATCH>
+__global__ __launch_bounds__(kFFTThreads, fft_waves(MAXN))
+void fft_analysis_kernel(const DevPlan *__restrict__ plans,
                                                                    CallArgs single,
                                                                    const CallArgs *__restrict__ calls,
                                                                    const Tile *__restrict__ tiles) {
@@ -818,17 +824,17 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
     fft_tile<BATCH>(rings, T, K, true, G);
     const FFTRing &R = G.R;
     const int N = R.N, mt = R.mt, ncol = G.ncol;
-    __builtin_assume(N >= 1 && N <= kFFTMaxRing);  // offsets within a ring fit scalar-base loads
+    __builtin_assume(N >= 1 && N <= MAXN);  // offsets within a ring fit scalar-base loads
     float2 *tw = smem;
     float2 *b0 = smem + N;
     const FFTPass pass0 = load_pass(as_global(tables.passes) + R.passes + (R.prime ? min(1, R.nf - 1) : 0));
-    Twiddles twr;
+    Twiddles<MAXN> twr;
     twr.load(tables.twiddle, R.tw_off, N, tid);
     const SHT_GLOBAL float *field = as_global(static_cast<const float *>(C.in)) + (long long)G.k0 * C.ld_in;
     const GridRings in{const_cast<SHT_GLOBAL float *>(field + R.ring_n), const_cast<SHT_GLOBAL float *>(field + R.ring_s),
                        C.ld_in, ncol};
     {
-        constexpr int U = (kFFTMaxRing + kFFTThreads - 1) / kFFTThreads;
+        constexpr int U = MAXN / kFFTThreads;
         // all loads of the thread in flight before the first LDS store (columns past ncol
         // re-read column 0 and are not stored)
         float vn[kFFTCols][U], vs[kFFTCols][U];
@@ -855,7 +861,7 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
         }
         __syncthreads();
     }
-    fft_run<false, false>(tables, R, b0, tw, N, mt, ncol, pass0, GridRings{}, tid);
+    fft_run<false, false, MAXN>(tables, R, b0, tw, N, mt, ncol, pass0, GridRings{}, tid);
     {
         SHT_GLOBAL float4 *fb = as_global(static_cast<float4 *>(C.fbuf)) + R.fboff * (long long)K + G.k0;
         int t = tid;
@@ -869,7 +875,7 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
         // first one of an order on
         const int mte = R.mte;
 #pragma unroll
-        for (int u = 0; u < kFFTRowPasses; ++u) {
+        for (int u = 0; u < fft_row_passes(MAXN); ++u) {
             const int mm = m0 + kFFTRowsPerPass * u;
             if (col >= ncol || mm > mte) continue;
             if (mm > mt) {
@@ -889,14 +895,21 @@ __global__ __launch_bounds__(kFFTThreads, 5) void fft_analysis_kernel(const DevP
 
 // ================================================================== entry points
 
-const void *fft_kernel(int stage, bool batch, bool accumulate) {
+template <int MAXN>
+static const void *fft_entry(int stage, bool batch, bool accumulate) {
     if (stage == kFFTSynthesis) {
-        if (accumulate && !batch) return reinterpret_cast<const void *>(&fft_synthesis_kernel<false, true>);
-        return batch ? reinterpret_cast<const void *>(&fft_synthesis_kernel<true>)
-                     : reinterpret_cast<const void *>(&fft_synthesis_kernel<false>);
+        if (accumulate && !batch) return reinterpret_cast<const void *>(&fft_synthesis_kernel<MAXN, false, true>);
+        return batch ? reinterpret_cast<const void *>(&fft_synthesis_kernel<MAXN, true>)
+                     : reinterpret_cast<const void *>(&fft_synthesis_kernel<MAXN, false>);
     }
-    return batch ? reinterpret_cast<const void *>(&fft_analysis_kernel<true>)
-                 : reinterpret_cast<const void *>(&fft_analysis_kernel<false>);
+    return batch ? reinterpret_cast<const void *>(&fft_analysis_kernel<MAXN, true>)
+                 : reinterpret_cast<const void *>(&fft_analysis_kernel<MAXN, false>);
+}
+
+const void *fft_kernel(int stage, bool batch, int cls, bool accumulate) {
+    if (cls == 0) return fft_entry<fft_class_ring(0)>(stage, batch, accumulate);
+    if (cls == 1) return fft_entry<fft_class_ring(1)>(stage, batch, accumulate);
+    return fft_entry<fft_class_ring(2)>(stage, batch, accumulate);
 }
 
 }  // namespace sht

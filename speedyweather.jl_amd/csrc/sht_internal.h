@@ -38,6 +38,11 @@ constexpr int kMaxFactors = 24;
 constexpr int kFFTThreads = 256;
 // Largest ring the FFT kernel takes, and columns per FFT workgroup.
 constexpr int kFFTMaxRing = 1024;
+// The FFT kernels are instantiated for rings of up to 256, 512 and kFFTMaxRing points (classes 0,
+// 1, 2): a thread's loads, the passes' column choices and the prime pass's row tiles, and with
+// them registers, code and workgroups per CU, follow the bound (figures in sht_fft.hip).
+constexpr int kFFTClasses = 3;
+constexpr int fft_class_ring(int cls) { return cls == 0 ? 256 : cls == 1 ? 512 : kFFTMaxRing; }
 constexpr int kFFTCols = 4;
 // A first radix of at least kMfmaMinPrime runs as the MFMA pass; the factorisation puts
 // every prime from kMfmaMinRadix up first (the largest one), and 11 or 13 first only when
@@ -51,6 +56,7 @@ constexpr int kMaxRegisterRadix = 13;
 // row tiles (16 output frequencies each) one wave holds for its column tile in a round.
 constexpr int kMaxMfmaRadix = 255;
 constexpr int kPrimeRowTiles = 4;
+constexpr int prime_row_tiles(int max_ring) { return max_ring <= 256 ? 1 : max_ring <= 512 ? 2 : kPrimeRowTiles; }
 // Row tiles per wave of the MFMA prime pass for radix r on M = N / r butterflies per column
 // and ncol columns, maximised over the rounds (host check of kPrimeRowTiles).
 inline int prime_rows_per_wave(int r, int M, int ncol) {
@@ -312,7 +318,7 @@ const void *legendre_kernel(int stage, int mode, bool batch);
 const void *legendre_mixed_kernel(int mode);  // single-call synthesis with CallArgs::mixed
 // accumulate: the single-call synthesis that adds into its output (pullbacks); batches
 // never accumulate.
-const void *fft_kernel(int stage, bool batch, bool accumulate = false);
+const void *fft_kernel(int stage, bool batch, int cls, bool accumulate = false);  // cls: ring class
 // Ring DFT on MFMA (sht_dft.hip): FP16 hi/lo or FP32 products, cg = 4 or 8 columns per
 // workgroup; single calls launch n * ceil(K / cg) blocks, dynamic LDS dft_smem_bytes.
 const void *dft_kernel(int stage, bool f16, int cg, bool batch, bool accumulate = false);

@@ -347,6 +347,7 @@ struct sht_plan {
     const DevPlan *dPv = nullptr;
     bool pol_ok[kPolicies] = {};  // the policy factorises every ring
     int pol = 0;                  // chosen policy
+    int fft_class = sht::kFFTClasses - 1;  // ring class of the FFT kernels
     std::vector<void *> allocs;
     // single-call Legendre launch orders, one per column-group count cgs = 1..max, grouped
     // by order m per XCD ([1]) or plain heavy-first ([0])
@@ -846,6 +847,20 @@ int build_plan(sht_plan *pl) {
         }
     }
     if (g.nlon_max > sht::kFFTMaxRing) return fail(SHT_ERR_UNSUPPORTED, "ring too long for the LDS FFT");
+    // the smallest ring class that holds every ring, and the prime pass's row tiles under every
+    // factorisation policy
+    for (int c = sht::kFFTClasses - 1; c >= 0; --c) {
+        bool ok = g.nlon_max <= sht::fft_class_ring(c);
+        for (int q = 0; q < kPolicies && ok; ++q)
+            for (int j = 0; j < n && pl->pol_ok[q] && ok; ++j) {
+                const int r = nfac_v[q][j] > 0 ? fac_v[q][(size_t)j * sht::kMaxFactors] : 0;
+                if (r < sht::kMfmaMinPrime || !(r & 1)) continue;
+                for (int ncol = 1; ncol <= sht::kFFTCols; ++ncol)
+                    ok = ok && sht::prime_rows_per_wave(r, g.nlon[j] / r, ncol) <=
+                                   sht::prime_row_tiles(sht::fft_class_ring(c));
+            }
+        if (ok) pl->fft_class = c;
+    }
     const int kg = sht::kFFTCols;
     P.kg = kg;
     P.fft_smem = (g.nlon_max + kg * g.nlon_max) * 8;  // twiddles + one in-place buffer
@@ -1092,9 +1107,9 @@ int build_plan(sht_plan *pl) {
     if (P.fft_smem > 65536) {
         for (bool b : {false, true})
             for (int st : {sht::kFFTSynthesis, sht::kFFTAnalysis})
-                (void)hipFuncSetAttribute(sht::fft_kernel(st, b), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          P.fft_smem);
-        (void)hipFuncSetAttribute(sht::fft_kernel(sht::kFFTSynthesis, false, true),
+                (void)hipFuncSetAttribute(sht::fft_kernel(st, b, pl->fft_class),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, P.fft_smem);
+        (void)hipFuncSetAttribute(sht::fft_kernel(sht::kFFTSynthesis, false, pl->fft_class, true),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, P.fft_smem);
     }
     const size_t fb_bytes = (size_t)g.fb_rows * d.nlayers * 16;
@@ -1319,11 +1334,11 @@ static StageLaunch plan_stage_launch(const sht_plan *plan, int stage, const Call
                         dim3(plan->g.n * ((K + cg - 1) / cg)), (unsigned)plan->dft_smem[syn][f16][cg == 8], nullptr};
             }
             if (stage == sht::kFFTSynthesis)
-                return {sht::fft_kernel(stage, false, c.accumulate != 0), dim3(fft_blocks(plan->g.n, K, c.paired != 0)),
-                        (unsigned)plan->P.fft_smem, reinterpret_cast<const Tile *>(plan->P.rings)};
+                return {sht::fft_kernel(stage, false, plan->fft_class, c.accumulate != 0),
+                        dim3(fft_blocks(plan->g.n, K, c.paired != 0)), (unsigned)plan->P.fft_smem, reinterpret_cast<const Tile *>(plan->P.rings)};
             // the FFT kernels of a single call take the ring records in place of a tile list
-            return {sht::fft_kernel(stage, false), dim3(fft_blocks(plan->g.n, K, true)), (unsigned)plan->P.fft_smem,
-                    reinterpret_cast<const Tile *>(plan->P.rings)};
+            return {sht::fft_kernel(stage, false, plan->fft_class), dim3(fft_blocks(plan->g.n, K, true)),
+                    (unsigned)plan->P.fft_smem, reinterpret_cast<const Tile *>(plan->P.rings)};
         }
         default:
             return {sht::legendre_kernel(stage, plan->d.precision, false), dim3(plan->nana[gx][cgs - 1]), 0,
@@ -2060,6 +2075,7 @@ struct sht_batch {
     const Tile *tiles[4] = {nullptr, nullptr, nullptr, nullptr};
     int ntiles[4] = {0, 0, 0, 0};
     unsigned fft_smem = 0;
+    int fft_class = 0;  // the largest ring class of its plans
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     bool use_graph = false;
@@ -2077,7 +2093,7 @@ void free_batch(sht_batch *b) {
 
 const void *stage_func(const sht_batch *b, int st) {
     return (st == sht::kLegendreSynthesis || st == sht::kLegendreAnalysis) ? sht::legendre_kernel(st, b->mode, true)
-                                                                            : sht::fft_kernel(st, true);
+                                                                            : sht::fft_kernel(st, true, b->fft_class);
 }
 
 int build_batch(sht_batch *b, const sht_batch_item *items, int n, int flags) {
@@ -2186,6 +2202,7 @@ int build_batch(sht_batch *b, const sht_batch_item *items, int n, int flags) {
     for (sht_plan *pl : plans) {
         dplans.push_back(pl->P);
         b->fft_smem = std::max<unsigned>(b->fft_smem, (unsigned)pl->P.fft_smem);
+        b->fft_class = std::max(b->fft_class, pl->fft_class);
     }
     if ((rc = dev_upload(b->allocs, dplans, &b->plans))) return rc;
     if ((rc = dev_upload(b->allocs, calls, &b->calls))) return rc;
@@ -2208,8 +2225,8 @@ int build_batch(sht_batch *b, const sht_batch_item *items, int n, int flags) {
     }
     if (b->fft_smem > 65536) {
         for (int st : {sht::kFFTSynthesis, sht::kFFTAnalysis})
-            (void)hipFuncSetAttribute(sht::fft_kernel(st, true), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)b->fft_smem);
+            (void)hipFuncSetAttribute(sht::fft_kernel(st, true, b->fft_class),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)b->fft_smem);
     }
     if (flags & SHT_BATCH_NO_GRAPH) return SHT_OK;
     // explicit graph: one kernel node per non-empty stage, chained in stage order
