@@ -140,20 +140,21 @@ __device__ __forceinline__ LegTile load_leg_tile(const Tile *tiles) {
 }
 
 // acc[t] += A_t (16 rows x 32 contraction, this lane's fragment of row tile t < TPW) x B
-// tile columns cb*16..cb*16+15 of parity p; each B fragment is read once for all TPW row
-// tiles.  FP32: af[t][8] holds the lane's A values of tile t for the 8 K-steps of 4.
+// tile columns cb*16..cb*16+15 of parity p for the column blocks cb = H, H + 1; each B fragment
+// is read once for all TPW row tiles.  half: the second half of the contraction is all zeros.  FP32: af[t][8] holds the lane's A values of tile t for the 8 K-steps of 4.
 // Split modes: ap[t][q] holds part q of the lane's A fragment; FP16 sums lo·hi, hi·lo,
 // hi·hi per chunk and adds the chunk rescaled, BF16 accumulates the six products of parts
 // (i, j) with i + j <= 2, smallest first.
-template <int MODE, int NCB, int TPW>
-__device__ inline void mma_chunk(const unsigned char *sm, int buf, int p, int row, int grp, const float (&af)[TPW][8],
-                                 const V8of<MODE> (&ap)[TPW][3], f4 (&acc)[TPW][NCB]) {
+template <int MODE, int H, int TPW>
+__device__ inline void mma_blocks(const unsigned char *sm, int buf, int p, int row, int grp, const float (&af)[TPW][8],
+                                 const V8of<MODE> (&ap)[TPW][3], f4 (&acc)[TPW][4], bool half = false) {
     if constexpr (MODE == kFP32) {
         const float *B = reinterpret_cast<const float *>(sm) + buf * kTileF + p * kColsReal * kRowF;
 #pragma unroll
         for (int ks = 0; ks < kChunk / 4; ++ks) {
+            if (ks == kChunk / 8 && half) break;  // uniform
 #pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) {
+            for (int cb = H; cb < H + 2; ++cb) {
                 const float b = B[(cb * 16 + row) * kRowF + 4 * ks + grp];
 #pragma unroll
                 for (int t = 0; t < TPW; ++t) acc[t][cb] = mfma_f32(af[t][ks], b, acc[t][cb]);
@@ -164,7 +165,7 @@ __device__ inline void mma_chunk(const unsigned char *sm, int buf, int p, int ro
         constexpr int NP = split_parts(MODE);
         const u16 *B0 = reinterpret_cast<const u16 *>(sm) + (buf * NP) * kTileH + p * kColsReal * kRowH;
 #pragma unroll
-        for (int cb = 0; cb < NCB; ++cb) {
+        for (int cb = H; cb < H + 2; ++cb) {
             const int col = cb * 16 + row;
             V8 b[NP];
 #pragma unroll
@@ -196,21 +197,21 @@ __device__ inline void mma_chunk(const unsigned char *sm, int buf, int p, int ro
 }
 
 // The same for one row tile.
-template <int MODE, int NCB>
-__device__ inline void mma_chunk1(const unsigned char *sm, int buf, int p, int row, int grp, const float (&af)[8],
-                                  const V8of<MODE> (&ap)[3], f4 (&acc)[NCB]) {
+template <int MODE, int H>
+__device__ inline void mma_blocks1(const unsigned char *sm, int buf, int p, int row, int grp, const float (&af)[8],
+                                  const V8of<MODE> (&ap)[3], f4 (&acc)[4]) {
     float a1[1][8];
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) a1[0][ks] = af[ks];
     V8of<MODE> p1[1][3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) p1[0][q] = ap[q];
-    f4 c1[1][NCB];
+    f4 c1[1][4];
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) c1[0][cb] = acc[cb];
-    mma_chunk<MODE, NCB, 1>(sm, buf, p, row, grp, a1, p1, c1);
+    for (int cb = H; cb < H + 2; ++cb) c1[0][cb] = acc[cb];
+    mma_blocks<MODE, H, 1>(sm, buf, p, row, grp, a1, p1, c1);
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) acc[cb] = c1[0][cb];
+    for (int cb = H; cb < H + 2; ++cb) acc[cb] = c1[0][cb];
 }
 
 // ============================================================ Legendre synthesis
@@ -272,6 +273,11 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
     const bool active = tile < Jt;
     const long long off = R.lm_off;
     const int kbase = cg * kColsComplex;
+    // The column blocks 2 and 3 hold columns.  The FP32 products take most of a workgroup's time
+    // (64 MFMAs of 32 cycles per wave and chunk), those of absent columns too: with them left
+    // out, T255 K=16 15.2 -> 11.4 us, T127 K=8 7.0 -> 5.7, T31 K=8 4.1 -> 3.7 (FP16x3: T255 K=16
+    // 11.0 -> 10.3); a call of full groups pays the branch (T127 K=32 7.5 -> 7.6).
+    const bool upper = (BATCH && cmap) || K - kbase > 16;
     const int row = lane & 15, grp = lane >> 4;
     // staging role
     const int kk = stage_column<MODE>(tid), g = tid & 7;
@@ -360,9 +366,24 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 4) void legendre_synthes
         load(nxt, c + 1);
         __syncthreads();
         if (active) {
-#pragma unroll
-            for (int p = 0; p < 2; ++p)
-                mma_chunk1<MODE, 4>(sm, buf, p, row, grp, cur.af[p], cur.ap[p], acc[p]);
+            auto blocks = [&](auto h, int p) {
+                mma_blocks1<MODE, h()>(sm, buf, p, row, grp, cur.af[p], cur.ap[p], acc[p]);
+            };
+            constexpr std::integral_constant<int, 0> lo;
+            constexpr std::integral_constant<int, 2> hi;
+            if constexpr (MODE == kFP32) {  // four accumulation chains in each half
+                blocks(lo, 0);
+                blocks(lo, 1);
+                if (upper) {
+                    blocks(hi, 0);
+                    blocks(hi, 1);
+                }
+            } else {  // one parity's operands at a time: both spill (T255 K=64 18.6 -> 22.6 us)
+                blocks(lo, 0);
+                if (upper) blocks(hi, 0);
+                blocks(lo, 1);
+                if (upper) blocks(hi, 1);
+            }
         }
     };
 
@@ -472,6 +493,10 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 3) void legendre_analysi
     const int lt0 = kAnaTiles * T.blk + TPW * (w >> 1);  // first degree tile of this wave
     const long long off = R.lm_off;
     const int kbase = cg * kColsComplex;
+    // The column blocks 2 and 3 hold columns (as in the synthesis: T255 K=16 15.2 -> 12.5 us,
+    // T127 K=8 5.2 -> 4.5, T31 K=8 3.2 -> 3.0).
+    const bool upper = (BATCH && cmap) || K - kbase > 16;
+    const bool active = 32 * lt0 + p < L;  // the wave's tiles hold degrees of the order
     const int row = lane & 15, grp = lane >> 4;
     const int kk = stage_column<MODE>(tid), g = tid & 7;
     bool kok = kbase + kk < K;
@@ -558,7 +583,14 @@ __global__ __launch_bounds__(256, MODE == kBF16x3 ? 2 : 3) void legendre_analysi
         stage4<MODE>(sm, buf, 1, kk, g, re, im);
         load(nxt, c + 1);
         __syncthreads();
-        mma_chunk<MODE, 4, TPW>(sm, buf, p, row, grp, cur.af, cur.ap, acc);
+        // idle waves and zero halves of the last chunk leave the matrix cores to the other
+        // workgroups: FP32 T127 K=392 27.0 -> 25.1 us, T255 K=64 25.4 -> 24.1 (the branch costs
+        // BF16x3 more than it saves: T255 K=16 13.2 -> 14.0)
+        if (MODE == kBF16x3 || active) {
+            const bool half = n - j0 - kChunk * c <= kChunk / 2;
+            mma_blocks<MODE, 0, TPW>(sm, buf, p, row, grp, cur.af, cur.ap, acc, half);
+            if (upper) mma_blocks<MODE, 2, TPW>(sm, buf, p, row, grp, cur.af, cur.ap, acc, half);
+        }
     };
 
     Ops S0, S1;
