@@ -115,35 +115,28 @@ struct FastDiv {
 };
 
 // U, V = (u, v) cos(lat) of packed coefficient lm on the unit sphere from the column's
-// vorticity and divergence (spectral_gradients.jl:331-366): a 3-point stencil in l.
+// vorticity and divergence (spectral_gradients.jl:331-366): a 3-point stencil in l.  The
+// neighbours are read whatever the degree, inside the column, and selected afterwards: a
+// branch on the degree would start them only when it has arrived (dry core's columns, 8 members
+// and levels: T31 3.7 -> 3.3 us, T127 9.5 -> 9.3).
 __device__ __forceinline__ void uv_stencil(const DevPlan &P, const SHT_GLOBAL float2 *vor, const SHT_GLOBAL float2 *dv,
                                            int lm, float2 &uu, float2 &vv) {
+    const int lo = max(lm - 1, 0), hi = min(lm + 1, P.nharm - 1);
+    const float2 z = gload(vor + lm), d = gload(dv + lm);
+    float2 zm = gload(vor + lo), dm = gload(dv + lo), zp = gload(vor + hi), dp = gload(dv + hi);
     const int l = as_global(P.l_of)[lm];
     const float x = as_global(P.uv_x)[lm], u1 = as_global(P.uv_1)[lm], u2 = as_global(P.uv_2)[lm];
-    const float2 z = gload(vor + lm), d = gload(dv + lm);
-    float2 du = make_float2(0.f, 0.f), dvv = make_float2(0.f, 0.f);
-    // i x D and i x ζ
-    if (lm == 0) {
-        float2 zp = make_float2(0.f, 0.f), dp = make_float2(0.f, 0.f);
-        if (P.lmax > 1) {
-            zp = gload(vor + 1);
-            dp = gload(dv + 1);
-        }
-        uu = make_float2(-x * d.y + u2 * zp.x, x * d.x + u2 * zp.y);
-        vv = make_float2(-x * z.y - u2 * dp.x, x * z.x - u2 * dp.y);
-    } else if (l == P.lmax - 1) {
-        const float2 zm = gload(vor + lm - 1), dm = gload(dv + lm - 1);
+    const bool first = lm == 0, last = !first && l == P.lmax - 1;
+    if (first) zm = dm = make_float2(0.f, 0.f);
+    // u2 is 0 on the second-to-last row, so the upper neighbours only enter below it
+    if (!(first ? P.lmax > 1 : l < P.lmax - 2)) zp = dp = make_float2(0.f, 0.f);
+    // i x D and i x ζ; the fused products are spelled out, as every result must round the same
+    // wherever this is inlined
+    uu = make_float2(fmaf(-u1, zm.x, fmaf(u2, zp.x, -(x * d.y))), fmaf(-u1, zm.y, fmaf(x, d.x, u2 * zp.y)));
+    vv = make_float2(fmaf(-u2, dp.x, fmaf(u1, dm.x, -(x * z.y))), fmaf(-u2, dp.y, fmaf(x, z.x, u1 * dm.y)));
+    if (last) {
         uu = make_float2(-u1 * zm.x, -u1 * zm.y);
         vv = make_float2(u1 * dm.x, u1 * dm.y);
-    } else {
-        const float2 zm = gload(vor + lm - 1), dm = gload(dv + lm - 1);
-        if (l < P.lmax - 2) {
-            du = gload(vor + lm + 1);
-            dvv = gload(dv + lm + 1);
-        }
-        // u2 is 0 on the second-to-last row, so du, dvv only enter below it
-        uu = make_float2(-x * d.y + u2 * du.x - u1 * zm.x, x * d.x + u2 * du.y - u1 * zm.y);
-        vv = make_float2(-x * z.y + u1 * dm.x - u2 * dvv.x, x * z.x + u1 * dm.y - u2 * dvv.y);
     }
 }
 
