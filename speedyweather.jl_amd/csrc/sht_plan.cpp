@@ -2124,17 +2124,17 @@ int build_batch(sht_batch *b, const sht_batch_item *items, int n, int flags) {
         const int K = it.K;
         const int cgs = (K + sht::kColsComplex - 1) / sht::kColsComplex;
         const int kgs = (K + pl->P.kg - 1) / pl->P.kg;
-        auto add_fft = [&](int st, int call) {  // tiles (call, ring rank, column group)
+        // Tiles (call, ring rank, column group); a call's column groups of a ring are one unit, so
+        // the ring's tables and the lines its groups share stay on one XCD: 64 uneven round trips
+        // of T31 to T255 965 us in units of two column groups, 946 so, 957 with the calls of a
+        // plan sharing a unit (fewer, larger units balance worse).
+        auto add_fft = [&](int st, int call) {
             const std::vector<int> &order = pl->h_ring_order_v[pl->pol];
-            for (int r = 0; r < (int)order.size(); ++r)
-                for (int q = 0; q < kgs; q += 2) {
-                    LaunchUnit u{0.0, {}};
-                    for (int h = q; h < std::min(q + 2, kgs); ++h) {
-                        u.tiles.push_back({call, r, h, 0});
-                        u.cost += pl->h_ring_cost_v[pl->pol][order[r]];
-                    }
-                    st_units[st].push_back(u);
-                }
+            for (int r = 0; r < (int)order.size(); ++r) {
+                LaunchUnit u{kgs * pl->h_ring_cost_v[pl->pol][order[r]], {}};
+                for (int h = 0; h < kgs; ++h) u.tiles.push_back({call, r, h, 0});
+                st_units[st].push_back(u);
+            }
         };
         // Legendre calls are grouped by plan (and unscale flag): after the loop, the calls of a
         // group share column groups (merged_groups below)
