@@ -257,6 +257,11 @@ int sht_dry_tendencies(sht_plan *plan, const sht_dry_model *model, const void *v
 int sht_dry_leapfrog(sht_plan *plan, int32_t nlayers, int32_t nmembers, const void *const *state,
                      const void *const *prev, const void *tend, const float *nu, const float *nu_div, double dt2,
                      double w1, double w2, void *filtered, void *next, void *stream);
+/* Both at once: sht_dry_leapfrog of the state with the tendencies sht_dry_tendencies gives,
+ * which are not stored (one pass over the state less); the same results. */
+int sht_dry_step(sht_plan *plan, const sht_dry_model *model, const void *const *state, const void *const *prev,
+                 const float *nu, const float *nu_div, double dt2, double w1, double w2, void *filtered, void *next,
+                 void *spec, void *grid, void *fields, void *stream);
 
 /* Learned column correction (an addition of this library; no reference counterpart): an MLP
  * 32 -> 128 -> 128 -> 32 with GELU per grid column (8 levels x {u, v, T, ln ps}), BF16

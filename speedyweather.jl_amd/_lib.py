@@ -31,7 +31,7 @@ EXPORTS = (
     "sht_grid2spec_pullback", "sht_divergence", "sht_laplace", "sht_gradient", "sht_plan_create_matrix",
     "sht_synthesis_laplace", "sht_analysis_laplace", "sht_time_stage", "sht_tune_cache_save",
     "sht_tune_cache_load", "sht_transform_static", "sht_plan_set_graphs", "sht_plan_graph_count",
-    "sht_dry_tendencies", "sht_dry_leapfrog",
+    "sht_dry_tendencies", "sht_dry_leapfrog", "sht_dry_step",
 )
 
 
@@ -107,6 +107,7 @@ def lib() -> C.CDLL:
         L.sht_batch_uses_graph.argtypes = [vp]
         L.sht_batch_destroy.argtypes = [vp]
         L.sht_dry_tendencies.argtypes = [vp, C.POINTER(ShtDryModel)] + [vp] * 8 + [i32, vp]
+        L.sht_dry_step.argtypes = [vp, C.POINTER(ShtDryModel)] + [vp] * 4 + [C.c_double] * 3 + [vp] * 6
         L.sht_dry_leapfrog.argtypes = [vp, i32, i32] + [vp] * 5 + [C.c_double] * 3 + [vp] * 3
         L.sht_mlp_create.argtypes = [i32, i32, C.POINTER(vp)]
         L.sht_mlp_set_params.argtypes = [vp, vp]

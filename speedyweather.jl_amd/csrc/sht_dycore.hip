@@ -4,8 +4,8 @@
 //
 // Every kernel is a single pass bound by memory (large ensembles) or by its launch (T31).
 // Written as array operations, a step was about 190 kernels of 2-7 us with the host issuing
-// them, 1.1 ms per step at T31 with 8 members; with these four kernels around the four of the
-// two transforms it is 58 us (T127, 8 members: 1.2 ms -> 0.195 ms).  The kernels keep the array
+// them, 1.1 ms per step at T31 with 8 members; with these kernels around the four of the
+// two transforms it is 47 us (T127, 8 members: 1.2 ms -> 0.19 ms).  The kernels keep the array
 // operations' rounding (no contraction to FMA), so a run stays what it was.
 #include <algorithm>
 
@@ -145,16 +145,33 @@ __global__ __launch_bounds__(256) void dry_grid_kernel(const float *__restrict__
     }
 }
 
+// Time step of one coefficient: new = (base + dt2 tend) / (1 + dt2 nu), and with a previous
+// state (base = b, else base = x) the Robert-Asselin-Williams filter of the present one, x.
+__device__ __forceinline__ void dry_step(float2 x, float2 b, float2 t, float damp, float dt2, float w1, float w2,
+                                         int filter, SHT_GLOBAL float2 *now1, SHT_GLOBAL float2 *next) {
+#pragma clang fp contract(off)
+    const float rd = 1.f / damp;
+    float2 y = make_float2((b.x + dt2 * t.x) * rd, (b.y + dt2 * t.y) * rd);
+    if (filter) {
+        const float2 d = make_float2(b.x - 2.f * x.x + y.x, b.y - 2.f * x.y + y.y);
+        gstore(now1, make_float2(x.x + w1 * d.x, x.y + w1 * d.y));
+        y = make_float2(y.x - w2 * d.x, y.y - w2 * d.y);
+    }
+    gstore(next, y);
+}
+
 // Spectral tendencies (columns: vorticity, divergence, temperature EL each, ln ps E) from the
 // analysed fields s (columns of dry_grid_kernel) and the temperature (geopotential, G L x L
 // with zeros below the diagonal).  One thread per coefficient and level.  LT levels known at
 // compile time: the temperatures of the levels below are all in flight at once (8 members and
 // levels: T31 5.2 -> 3.8 us, T127 13.6 -> 12.7); LT = 0: L levels, one load after another.
-template <int LT>
+// STEP: the tendencies are not stored but applied (dry_step), one pass over the state instead of
+// two (8 members and levels: T31 3.8 + 3.4 -> 4.8 us, T127 12.7 + 12.4 -> 19.6).
+template <int LT, bool STEP>
 __global__ __launch_bounds__(256) void dry_tendency_kernel(const DevPlan *__restrict__ PP, const float2 *__restrict__ s_,
                                                            const float2 *__restrict__ temp_,
                                                            const float *__restrict__ G_, float2 *__restrict__ tend_,
-                                                           int Lrt, int E, float radius, float radius2) {
+                                                           int Lrt, int E, float radius, float radius2, DryStep S) {
 #pragma clang fp contract(off)
     const int L = LT > 0 ? LT : Lrt;
     const DevPlan &P = *PP;
@@ -165,12 +182,30 @@ __global__ __launch_bounds__(256) void dry_tendency_kernel(const DevPlan *__rest
     SHT_GLOBAL float2 *tend = as_global(tend_) + lm;
     const int l = as_global(P.l_of)[lm];
     const float keep = l == P.lmax - 1 ? 0.f : 1.f;  // the extra degree has no prognostic tendency
+    // tendency t of prognostic field f, column `row` of all
+    auto put = [&](int f, long long row, float2 t, float2 x, float2 b) {
+        if constexpr (STEP) {
+            const float damp = f == 3 ? 1.f : 1.f + S.dt2 * (f == 1 ? as_global(S.nu_div) : as_global(S.nu))[lm];
+            dry_step(x, b, t, damp, S.dt2, S.w1, S.w2, S.filter, as_global(S.now1) + lm + row * nh,
+                     as_global(S.next) + lm + row * nh);
+        } else {
+            gstore(tend + row * nh, t);
+        }
+    };
+    auto state = [&](const float2 *now, const float2 *prev, long long col, float2 &x, float2 &b) {
+        if constexpr (STEP) {
+            x = b = gload(as_global(now) + lm + col * nh);
+            if (S.filter) b = gload(as_global(prev) + lm + col * nh);  // uniform
+        }
+    };
     for (int row = blockIdx.y; row < EL + E; row += gridDim.y) {
         if (row >= EL) {
             const int e = row - (int)EL;
             const float2 q = gload(s + (6 * EL + e) * nh);
             const float w = lm == 0 ? 0.f : keep;  // mass conservation: the mean of ln ps stays
-            gstore(tend + (3 * EL + e) * nh, make_float2(q.x * w, q.y * w));
+            float2 x = q, b = q;
+            state(S.now.lnps, S.prev.lnps, e, x, b);
+            put(3, 3 * EL + e, make_float2(q.x * w, q.y * w), x, b);
             continue;
         }
         const int e = row / L, k = row - e * L;
@@ -186,6 +221,10 @@ __global__ __launch_bounds__(256) void dry_tendency_kernel(const DevPlan *__rest
         const float2 ke = gload(a + EL * nh), Tt = gload(a + 2 * EL * nh);
         const float4 gy = gload(as_global(P.gy) + lm);  // gy.x, gy.y, gx.x are zero at the last degree
         const float mx = gload(as_global(P.gx) + lm).x;
+        float2 xz = u, bz = u, xd = u, bd = u, xt = u, bt = u;
+        state(S.now.vor, S.prev.vor, row, xz, bz);
+        state(S.now.div, S.prev.div, row, xd, bd);
+        state(S.now.temp, S.prev.temp, row, xt, bt);
         float2 phi = make_float2(0.f, 0.f);
         const SHT_GLOBAL float2 *T = as_global(temp_) + (long long)e * L * nh + lm;
         const SHT_GLOBAL float *G = as_global(G_) + k * L;
@@ -215,16 +254,14 @@ __global__ __launch_bounds__(256) void dry_tendency_kernel(const DevPlan *__rest
         const float2 divT = make_float2(iuT.x - gy.x * vTm.x + gy.y * vTp.x, iuT.y - gy.x * vTm.y + gy.y * vTp.y);
         const float eig = -(float)l * (float)(l + 1);
         const float2 lap = make_float2(eig * (phi.x + ke.x), eig * (phi.y + ke.y));
-        gstore(tend + row * nh, make_float2(curl.x * ri * keep, curl.y * ri * keep));
-        gstore(tend + (EL + row) * nh,
-               make_float2((div.x * ri - lap.x * rr) * keep, (div.y * ri - lap.y * rr) * keep));
-        gstore(tend + (2 * EL + row) * nh, make_float2((-divT.x * ri + Tt.x) * keep, (-divT.y * ri + Tt.y) * keep));
+        put(0, row, make_float2(curl.x * ri * keep, curl.y * ri * keep), xz, bz);
+        put(1, EL + row, make_float2((div.x * ri - lap.x * rr) * keep, (div.y * ri - lap.y * rr) * keep), xd, bd);
+        put(2, 2 * EL + row, make_float2((-divT.x * ri + Tt.x) * keep, (-divT.y * ri + Tt.y) * keep), xt, bt);
     }
 }
 
-// Time step of every prognostic column: new = (base + dt2 tend) / (1 + dt2 nu), and with a
-// previous state the Robert-Asselin-Williams filter of the present one.  Outputs: columns as
-// the tendencies'.
+// Time step of every prognostic column from stored tendencies (a correction may have changed
+// them).  Outputs: columns as the tendencies'.
 __global__ __launch_bounds__(256) void dry_leapfrog_kernel(DryState now, DryState prev, const float2 *__restrict__ tend_,
                                                            const float *__restrict__ nu_,
                                                            const float *__restrict__ nu_div_, float2 *__restrict__ now1_,
@@ -241,14 +278,7 @@ __global__ __launch_bounds__(256) void dry_leapfrog_kernel(DryState now, DryStat
         float2 b = x;
         if (filter) b = gload(as_global(f == 0 ? prev.vor : f == 1 ? prev.div : f == 2 ? prev.temp : prev.lnps) + in);
         const float damp = f == 3 ? 1.f : 1.f + dt2 * (f == 1 ? as_global(nu_div_) : as_global(nu_))[lm];
-        const float rd = 1.f / damp;
-        float2 y = make_float2((b.x + dt2 * t.x) * rd, (b.y + dt2 * t.y) * rd);
-        if (filter) {
-            const float2 d = make_float2(b.x - 2.f * x.x + y.x, b.y - 2.f * x.y + y.y);
-            gstore(as_global(now1_) + out, make_float2(x.x + w1 * d.x, x.y + w1 * d.y));
-            y = make_float2(y.x - w2 * d.x, y.y - w2 * d.y);
-        }
-        gstore(as_global(next_) + out, y);
+        dry_step(x, b, t, damp, dt2, w1, w2, filter, as_global(now1_) + out, as_global(next_) + out);
     }
 }
 
@@ -274,18 +304,24 @@ int launch_dry_grid(const float *g, float *fields, const float *coslat_inv, cons
     return (int)hipGetLastError();
 }
 
+template <bool STEP>
+static int launch_tendency(const DevPlan *P, int nharm, const void *s, const float2 *temp, const float *G, void *tend,
+                           int L, int E, double radius, const DryStep &S, void *stream) {
+    const dim3 grid((nharm + 255) / 256, std::min(E * L + E, kMaxGridY));
+    auto *f = L == 8 ? &dry_tendency_kernel<8, STEP> : &dry_tendency_kernel<0, STEP>;
+    f<<<grid, 256, 0, as_stream(stream)>>>(P, static_cast<const float2 *>(s), temp, G, static_cast<float2 *>(tend), L, E,
+                                           (float)radius, (float)(radius * radius), S);
+    return (int)hipGetLastError();
+}
+
 int launch_dry_tendency(const DevPlan *P, int nharm, const void *s, const float2 *temp, const float *G, void *tend, int L,
                         int E, double radius, void *stream) {
-    const dim3 grid((nharm + 255) / 256, std::min(E * L + E, kMaxGridY));
-    if (L == 8)
-        dry_tendency_kernel<8><<<grid, 256, 0, as_stream(stream)>>>(P, static_cast<const float2 *>(s), temp, G,
-                                                                    static_cast<float2 *>(tend), L, E, (float)radius,
-                                                                    (float)(radius * radius));
-    else
-        dry_tendency_kernel<0><<<grid, 256, 0, as_stream(stream)>>>(P, static_cast<const float2 *>(s), temp, G,
-                                                                    static_cast<float2 *>(tend), L, E, (float)radius,
-                                                                    (float)(radius * radius));
-    return (int)hipGetLastError();
+    return launch_tendency<false>(P, nharm, s, temp, G, tend, L, E, radius, DryStep{}, stream);
+}
+
+int launch_dry_step(const DevPlan *P, int nharm, const void *s, const float *G, const DryStep &S, int L, int E,
+                    double radius, void *stream) {
+    return launch_tendency<true>(P, nharm, s, S.now.temp, G, nullptr, L, E, radius, S, stream);
 }
 
 int launch_dry_leapfrog(int nharm, const DryState &now, const DryState &prev, const void *tend, const float *nu,

@@ -1643,22 +1643,20 @@ static int check_dry(sht_plan *plan, int32_t L, int32_t E) {
     return SHT_OK;
 }
 
-int sht_dry_tendencies(sht_plan *plan, const sht_dry_model *model, const void *vor, const void *div, const void *temp,
-                       const void *lnps, void *tend, void *spec, void *grid, void *fields, int32_t with_grid,
-                       void *stream) {
-    sht::TraceRange trace_range("sht_dry_tendencies");
+// A state's analysed tendency fields in spec, then the spectral tendencies into tend, or with
+// `step` the time step.
+static int dry_tendencies(sht_plan *plan, const sht_dry_model *model, const sht::DryState &st, void *tend, void *spec,
+                          void *grid, void *fields, int32_t with_grid, const sht::DryStep *step, void *stream) {
     if (!model) return fail(SHT_ERR_ARG, "null model");
     const int L = model->nlayers, E = model->nmembers;
     int rc = check_dry(plan, L, E);
     if (rc) return rc;
-    if (!vor || !div || !temp || !lnps || !tend || !spec || !grid || !fields || !model->coslat_inv ||
-        !model->coriolis || !model->geopotential)
+    if (!st.vor || !st.div || !st.temp || !st.lnps || !(tend || step) || !spec || !grid || !fields ||
+        !model->coslat_inv || !model->coriolis || !model->geopotential)
         return fail(SHT_ERR_ARG, "null data pointer");
     if (!(model->radius > 0)) return fail(SHT_ERR_ARG, "radius must be positive");
     const int nharm = plan->g.nharm, np = (int)plan->g.npoints;
     const int down = 5 * E * L + (with_grid ? 3 : 2) * E, up = 6 * E * L + E;
-    const sht::DryState st{static_cast<const float2 *>(vor), static_cast<const float2 *>(div),
-                           static_cast<const float2 *>(temp), static_cast<const float2 *>(lnps)};
     DeviceGuard guard(plan->d.device);
     if ((rc = check_call(plan, spec, grid, std::max(down, up)))) return rc;
     auto launched = [](int e, const char *what) {
@@ -1675,9 +1673,39 @@ int sht_dry_tendencies(sht_plan *plan, const sht_dry_model *model, const void *v
                   "dry grid tendencies");
     if (rc) return rc;
     if ((rc = run_analysis(plan, fields, np, spec, nharm, up, 0, 0, 0, stream))) return rc;
+    if (step)
+        return launched(sht::launch_dry_step(plan->dP, nharm, spec, model->geopotential, *step, L, E, model->radius,
+                                             stream),
+                        "dry step");
     return launched(sht::launch_dry_tendency(plan->dP, nharm, spec, st.temp, model->geopotential, tend, L, E,
                                              model->radius, stream),
                     "dry spectral tendencies");
+}
+
+static sht::DryState dry_columns(const void *const *p) {
+    return sht::DryState{static_cast<const float2 *>(p[0]), static_cast<const float2 *>(p[1]),
+                         static_cast<const float2 *>(p[2]), static_cast<const float2 *>(p[3])};
+}
+
+int sht_dry_tendencies(sht_plan *plan, const sht_dry_model *model, const void *vor, const void *div, const void *temp,
+                       const void *lnps, void *tend, void *spec, void *grid, void *fields, int32_t with_grid,
+                       void *stream) {
+    sht::TraceRange trace_range("sht_dry_tendencies");
+    const void *const st[4] = {vor, div, temp, lnps};
+    return dry_tendencies(plan, model, dry_columns(st), tend, spec, grid, fields, with_grid, nullptr, stream);
+}
+
+int sht_dry_step(sht_plan *plan, const sht_dry_model *model, const void *const *state, const void *const *prev,
+                 const float *nu, const float *nu_div, double dt2, double w1, double w2, void *filtered, void *next,
+                 void *spec, void *grid, void *fields, void *stream) {
+    sht::TraceRange trace_range("sht_dry_step");
+    if (!state || !nu || !nu_div || !next || (prev && !filtered)) return fail(SHT_ERR_ARG, "null data pointer");
+    for (int i = 0; prev && i < 4; ++i)
+        if (!prev[i]) return fail(SHT_ERR_ARG, "null data pointer");
+    const sht::DryState now = dry_columns(state);
+    const sht::DryStep step{now, prev ? dry_columns(prev) : now, nu, nu_div, static_cast<float2 *>(filtered),
+                            static_cast<float2 *>(next), (float)dt2, (float)w1, (float)w2, prev ? 1 : 0};
+    return dry_tendencies(plan, model, now, nullptr, spec, grid, fields, 0, &step, stream);
 }
 
 int sht_dry_leapfrog(sht_plan *plan, int32_t nlayers, int32_t nmembers, const void *const *state,
@@ -1689,12 +1717,8 @@ int sht_dry_leapfrog(sht_plan *plan, int32_t nlayers, int32_t nmembers, const vo
     if (!state || !tend || !nu || !nu_div || !next || (prev && !filtered)) return fail(SHT_ERR_ARG, "null data pointer");
     for (int i = 0; i < 4; ++i)
         if (!state[i] || (prev && !prev[i])) return fail(SHT_ERR_ARG, "null data pointer");
-    auto columns = [](const void *const *p) {
-        return sht::DryState{static_cast<const float2 *>(p[0]), static_cast<const float2 *>(p[1]),
-                             static_cast<const float2 *>(p[2]), static_cast<const float2 *>(p[3])};
-    };
     DeviceGuard guard(plan->d.device);
-    rc = sht::launch_dry_leapfrog(plan->g.nharm, columns(state), columns(prev ? prev : state), tend, nu, nu_div,
+    rc = sht::launch_dry_leapfrog(plan->g.nharm, dry_columns(state), dry_columns(prev ? prev : state), tend, nu, nu_div,
                                   filtered, next, nlayers, nmembers, (float)dt2, (float)w1, (float)w2, prev ? 1 : 0,
                                   stream);
     if (rc) return fail(SHT_ERR_HIP, std::string("dry leapfrog launch: ") + hipGetErrorString((hipError_t)rc));

@@ -218,19 +218,27 @@ class DryPrimitiveModel:
     def _vector(self, x: torch.Tensor) -> torch.Tensor:
         return x.to(device=self.coslat.device, dtype=torch.float32).contiguous()
 
+    def _model(self):
+        """The model's descriptor and the tensors it points to."""
+        tables = [self._vector(t) for t in (self.coslat_inv, self.f, self.G)]
+        return ShtDryModel(self.L, self.E, self.a, R_DRY, KAPPA, *(t.data_ptr() for t in tables)), tables
+
+    def _work(self, with_grid: bool):
+        """The arrays between the kernels of a tendency: spectral columns, grid, grid tendencies."""
+        E, EL, npts, dev = self.E, self.E * self.L, self.grid.npoints, self.coslat.device
+        down, up = 5 * EL + (3 if with_grid else 2) * E, 6 * EL + E
+        return (torch.empty((max(5 * EL + 3 * E, up), self.spectrum.nharm), dtype=torch.complex64, device=dev),
+                torch.empty((down, npts), device=dev), torch.empty((up, npts), device=dev))
+
     def tendencies(self, st: dict, with_grid: bool = False):
         """Spectral tendencies of vor, div, temp (E*L, nharm) and lnps (E, nharm); with_grid
         also u, v, T (E, L, npoints) and lnps (E, 1, npoints)."""
         L, E = self.L, self.E
-        EL, n, npts, dev = E * L, self.spectrum.nharm, self.grid.npoints, self.coslat.device
+        EL, n, dev = E * L, self.spectrum.nharm, self.coslat.device
         ptr, keep = self._columns(st, "state")
-        tables = [self._vector(t) for t in (self.coslat_inv, self.f, self.G)]
-        model = ShtDryModel(L, E, self.a, R_DRY, KAPPA, *(t.data_ptr() for t in tables))
-        down, up = 5 * EL + (3 if with_grid else 2) * E, 6 * EL + E
+        model, tables = self._model()
         tend = torch.empty((3 * EL + E, n), dtype=torch.complex64, device=dev)
-        spec = torch.empty((max(5 * EL + 3 * E, up), n), dtype=torch.complex64, device=dev)
-        g = torch.empty((down, npts), device=dev)
-        fields = torch.empty((up, npts), device=dev)
+        spec, g, fields = self._work(with_grid)
         check(lib().sht_dry_tendencies(self.S._plan, C.byref(model), *ptr, tend.data_ptr(), spec.data_ptr(),
                                        g.data_ptr(), fields.data_ptr(), int(bool(with_grid)), self.S._stream()),
               "sht_dry_tendencies")
@@ -245,17 +253,21 @@ class DryPrimitiveModel:
     def step(self, correction=None):
         """One leapfrog step (Euler forward for the first); `correction(model, tend, grid)`
         may add to the spectral tendencies."""
-        need_grid = correction is not None
-        out = self.tendencies(self.state, with_grid=need_grid)
-        tend, grid = (out if need_grid else (out, None))
-        if correction is not None:
-            correction(self, tend, grid)
+        # without a correction the tendencies go straight into the step, unless a subclass or an
+        # instance has its own, or the class was given another
+        fused = correction is None and "tendencies" not in vars(self) and type(self).tendencies is _TENDENCIES
         L, E, n, dev = self.L, self.E, self.spectrum.nharm, self.coslat.device
         rows = 3 * E * L + E
-        tptr, tkeep = self._columns(tend, "tendency")
-        if any(p != tptr[0] + 8 * n * E * L * i for i, p in enumerate(tptr)):  # a correction put its own tensors there
-            tkeep = torch.cat(tkeep)
-            tptr = [tkeep.data_ptr()]
+        if not fused:
+            need_grid = correction is not None
+            out = self.tendencies(self.state, with_grid=need_grid)
+            tend, grid = (out if need_grid else (out, None))
+            if correction is not None:
+                correction(self, tend, grid)
+            tptr, tkeep = self._columns(tend, "tendency")
+            if any(p != tptr[0] + 8 * n * E * L * i for i, p in enumerate(tptr)):  # a correction put its own tensors there
+                tkeep = torch.cat(tkeep)
+                tptr = [tkeep.data_ptr()]
         sptr, skeep = self._columns(self.state, "state")
         nu, nu_div = self._vector(self.nu), self._vector(self.nu_div)
         arr = C.c_void_p * 4
@@ -268,9 +280,16 @@ class DryPrimitiveModel:
             dt2, prev = 2.0 * self.dt, arr(*pptr)
         w1 = self.robert * self.williams / 2
         w2 = self.robert * (1 - self.williams) / 2
-        check(lib().sht_dry_leapfrog(self.S._plan, L, E, arr(*sptr), prev, tptr[0], nu.data_ptr(), nu_div.data_ptr(),
-                                     dt2, w1, w2, None if filtered is None else filtered.data_ptr(), new.data_ptr(),
-                                     self.S._stream()), "sht_dry_leapfrog")
+        out = (None if filtered is None else filtered.data_ptr(), new.data_ptr())
+        if fused:
+            model, tables = self._model()
+            spec, g, fields = self._work(False)
+            check(lib().sht_dry_step(self.S._plan, C.byref(model), arr(*sptr), prev, nu.data_ptr(), nu_div.data_ptr(),
+                                     dt2, w1, w2, *out, spec.data_ptr(), g.data_ptr(), fields.data_ptr(),
+                                     self.S._stream()), "sht_dry_step")
+        else:
+            check(lib().sht_dry_leapfrog(self.S._plan, L, E, arr(*sptr), prev, tptr[0], nu.data_ptr(),
+                                         nu_div.data_ptr(), dt2, w1, w2, *out, self.S._stream()), "sht_dry_leapfrog")
         self.state_prev = self.state if filtered is None else self._split(filtered)
         self.state = self._split(new)
         self.nsteps += 1
@@ -322,3 +341,6 @@ class DryPrimitiveModel:
 
     def close(self):
         self.S.close()
+
+
+_TENDENCIES = DryPrimitiveModel.tendencies  # what step() may fuse with the time step

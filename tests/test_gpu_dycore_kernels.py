@@ -123,3 +123,33 @@ def test_bad_states_raise(sw, gpu):
     with pytest.raises(ValueError):
         m.tendencies({**st, "div": st["div"].cpu()})
     m.close()
+
+
+@pytest.mark.parametrize("L,E,trunc", [(8, 2, 31), (3, 3, 21), (1, 1, 30)])
+def test_fused_step_is_the_step_of_the_tendencies(sw, gpu, L, E, trunc):
+    """A step without a correction (tendencies applied where they are computed) gives bit for
+    bit what a step with a correction that changes nothing gives."""
+    m, w = (sw.dycore.DryPrimitiveModel(trunc, L, nmembers=E) for _ in range(2))
+    st = state(sw, m, 3 * trunc + L)
+    m.set_state(st)
+    w.set_state(st)
+    for _ in range(3):  # Euler, then two leapfrog steps with the filter
+        m.step()
+        w.step(correction=lambda model, tend, grid: None)
+        for k in st:
+            assert torch.equal(m.state[k], w.state[k]), k
+            assert torch.equal(m.state_prev[k], w.state_prev[k]), k
+    m.close()
+    w.close()
+
+
+def test_own_tendencies_are_used(sw, gpu):
+    class Still(sw.dycore.DryPrimitiveModel):
+        def tendencies(self, st, with_grid=False):
+            return {k: torch.zeros_like(v) for k, v in st.items()}
+    m = Still(21, 3, nmembers=1)
+    st = state(sw, m, 5)
+    m.set_state(st)
+    m.step()
+    assert torch.equal(m.state["lnps"], st["lnps"])
+    m.close()
