@@ -12,6 +12,12 @@
 // the next chunk's operands are loaded into registers while the current chunk's MFMAs
 // run, and the staged operand tile in LDS is double-buffered (one barrier per chunk).
 //
+// Bound by latency: little more than one workgroup per slot, each a chain of record load, first
+// operands, 1 to 6 chunk steps and stores; in FP32 then by the MFMAs (at most 62 % of their
+// rate).  Hence one record with everything the first loads need, no branch before them, and
+// 16-byte row stores: T255 K=64 synthesis / analysis FP16x3 20.9 / 23.0 -> 18.6 / 20.4 us, FP32
+// 28.7 / 29.6 -> 25.3 / 25.5; then the products no output needs are left out (below).
+//
 // Fourier buffer (the scratch of the call's stream): row (fboff[j] + m) holds, for every column k, a
 // float4 (N.re, N.im, S.re, S.im).  Synthesis writes the northern/southern Legendre sums
 // g_N, g_S there (legendre.jl:84-91); analysis reads the even/odd combinations

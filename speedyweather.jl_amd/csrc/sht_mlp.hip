@@ -131,8 +131,9 @@ __global__ __launch_bounds__(256) void mlp_forward_kernel(const bf16 *__restrict
 // L = mean((y - t)^2) over B x 32 values: forward, backward and the weight gradients of a
 // range of 32-row tiles in one workgroup of 8 waves.  In the chain of layers wave (rg, fg)
 // takes row group rg (16 rows) and the 32 features fg of every hidden layer; activations and
-// gradients pass between the waves of a row group through LDS, row-major (N tiles).  For the weight gradients, whose contraction runs over the 32
-// rows, they are also kept feature-major (F tiles): wave w owns output tile w of W2 and W1
+// gradients pass between the waves of a row group through LDS, row-major (N tiles).  For the
+// weight gradients, whose contraction runs over the 32 rows, they are also kept feature-major
+// (F tiles): wave w owns output tile w of W2 and W1
 // and input tile w of W3, accumulated over all tiles of the workgroup; the bias gradients are
 // products with ones.  Each workgroup writes one partial parameter gradient (99 KiB): one
 // 32-row tile per workgroup up to 256 workgroups (one per CU), then more tiles each.  Bound by
