@@ -810,10 +810,8 @@ void fft_synthesis_kernel(const DevPlan *__restrict__ plans, CallArgs single, co
 // and stored as (f_N + f_S, f_N - f_S) for orders 0..mt.
 template <int MAXN, bool BATCH>
 __global__ __launch_bounds__(kFFTThreads, fft_waves(MAXN))
-void fft_analysis_kernel(const DevPlan *__restrict__ plans,
-                                                                   CallArgs single,
-                                                                   const CallArgs *__restrict__ calls,
-                                                                   const Tile *__restrict__ tiles) {
+void fft_analysis_kernel(const DevPlan *__restrict__ plans, CallArgs single, const CallArgs *__restrict__ calls,
+                         const Tile *__restrict__ tiles) {
     extern __shared__ float4 smem4[];
     float2 *smem = reinterpret_cast<float2 *>(smem4);
     const int tid = threadIdx.x;
