@@ -852,6 +852,7 @@ void fft_analysis_kernel(const DevPlan *__restrict__ plans, CallArgs single, con
                 vs[c][u] = fs[i];
             }
         }
+        if (!BATCH && R.j < 0) return;  // padding of the launch order
         __builtin_amdgcn_sched_barrier(0);
         twr.store(tw, N, tid);
 #pragma unroll
