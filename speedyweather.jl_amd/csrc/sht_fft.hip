@@ -852,7 +852,6 @@ void fft_analysis_kernel(const DevPlan *__restrict__ plans, CallArgs single, con
                 vs[c][u] = fs[i];
             }
         }
-        if (!BATCH && R.j < 0) return;  // padding of the launch order
         __builtin_amdgcn_sched_barrier(0);
         twr.store(tw, N, tid);
 #pragma unroll
@@ -865,6 +864,9 @@ void fft_analysis_kernel(const DevPlan *__restrict__ plans, CallArgs single, con
         }
         __syncthreads();
     }
+    // padding of the launch order leaves here, the whole workgroup (ahead of the LDS stores the exit
+    // costs the other workgroups' schedule: T255 K=64 28.8 us instead of 28.1)
+    if (!BATCH && R.j < 0) return;
     fft_run<false, false, MAXN>(tables, R, b0, tw, N, mt, ncol, pass0, GridRings{}, tid);
     {
         SHT_GLOBAL float4 *fb = as_global(static_cast<float4 *>(C.fbuf)) + R.fboff * (long long)K + G.k0;
