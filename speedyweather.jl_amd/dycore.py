@@ -35,6 +35,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import operator
 
 import numpy as np
 import torch
@@ -50,6 +51,9 @@ GRAVITY = 9.81          # m/s^2
 R_DRY = 287.05          # J/kg/K
 CP = 1004.0             # J/kg/K
 KAPPA = R_DRY / CP
+
+
+_version, _requires_grad = operator.attrgetter("_version"), operator.attrgetter("requires_grad")
 
 
 def _eps(l, m):
@@ -121,8 +125,14 @@ def grid_latitudes(grid) -> np.ndarray:
 class DryPrimitiveModel:
     """Dry primitive equations at spectral truncation `trunc` (0-based, e.g. 31 or 127) on
     the octahedral Gaussian grid with quadratic dealiasing, `nlayers` sigma levels, for
-    `nmembers` independent states side by side (columns of every transform)."""
+    `nmembers` independent states side by side (columns of every transform).
 
+    A subclass may override `tendencies`, `uv`, `synth`, `analyse` and `_diffuse`, and the
+    tables (sigma levels, G, f, nu, ops, ...) may be replaced or written to: the step follows
+    them, as array operations instead of the library's kernels where these have the original
+    built in."""
+
+    @torch.inference_mode(False)  # its tables count writes, whatever mode it is built in
     def __init__(self, trunc: int, nlayers: int = 8, nmembers: int = 1, dt: float | None = None,
                  precision: str = "fp32", device="cuda:0", radius: float = RADIUS):
         self.device = torch.device(device)
@@ -166,6 +176,12 @@ class DryPrimitiveModel:
         self.state_prev = None
         self.state = None
         self.nsteps = 0
+        self._dev = self.coslat.device
+        # what the kernels have built in, to see that it is unchanged: each table and its count
+        # of in-place writes
+        self._levels = (L, self.dsigma)
+        self._built = self._tables()
+        self._writes = list(map(_version, self._built))
 
     # ------------------------------------------------------------------ transforms
     def _lta(self, t):
@@ -191,32 +207,82 @@ class DryPrimitiveModel:
         return U, V
 
     # ------------------------------------------------------------------ dynamics
-    def _columns(self, st: dict, what: str):
+    # The equations are written twice: as array operations (_tendencies_arrays, _diffuse, the
+    # last part of step), which take whatever torch takes, and as the library's kernels, 6 to 24
+    # times faster (8 members and levels: T127 1.2 -> 0.19 ms per step, T31 1.1 -> 0.05), which
+    # read raw memory of one form.  The kernels run where the model is as it was built
+    # (_kernels) and the tensors have that form (_plain, _columns); both give the same values.
+    # A step spends its host time on these checks, so each looks at a thing once.
+    @staticmethod
+    def _plain(t, shape) -> bool:
+        """t is memory: a tensor of that shape with nothing to differentiate (nor to map
+        through: _untraced)."""
+        return (type(t) in _TENSORS and t.shape == shape and not (t.requires_grad and torch.is_grad_enabled()))
+
+    @staticmethod
+    def _untraced() -> bool:
+        """No transform of functions (vmap, jvp, ...) and no forward differentiation is on."""
+        return torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+
+    def _tables(self) -> tuple:
+        return (self.sigma_half, self.sigma_full, self.G, *vars(self.ops).values())
+
+    def _kernels(self) -> bool:
+        """The library's kernels state this model: nothing that they have built in was replaced
+        or written to (sigma levels, geopotential matrix, operators, transforms, methods), and
+        the tables that they read hold one real value per grid point."""
+        S, grid, tables = self.S, (self.grid.npoints,), self._tables()
+        return (self._untraced()
+                and _methods(type(self)) == _METHODS_AS_BUILT and _METHODS.isdisjoint(vars(self))
+                and type(self.ops) is SpectralOps and _operators(SpectralOps) == _OPERATORS_AS_BUILT
+                and isinstance(self.dsigma, float) and (self.L, self.dsigma) == self._levels
+                and len(tables) == len(self._built) and all(map(operator.is_, tables, self._built))
+                and list(map(_version, tables)) == self._writes
+                and not (torch.is_grad_enabled() and any(map(_requires_grad, tables)))
+                and type(S) is SpectralTransform and S.spectrum == self.spectrum and S.grid == self.grid
+                and S.nlayers >= self.E * max(6 * self.L + 1, 5 * self.L + 3) and S.device == self._dev.index
+                and isinstance(self.a, (int, float)) and self.a > 0
+                and self._plain(self.f, grid) and self._plain(self.coslat_inv, grid)
+                and not self.f.is_complex() and not self.coslat_inv.is_complex())
+
+    def _columns(self, st: dict):
         """Device pointers of a state's vor, div, temp (E*L, nharm) and lnps (E, nharm), and the
-        tensors that hold them."""
+        tensors that hold them; None where a tensor has another form."""
         E, EL, n = self.E, self.E * self.L, self.spectrum.nharm
         keep, ptr = [], []
         for name, rows in (("vor", EL), ("div", EL), ("temp", EL), ("lnps", E)):
-            t = st[name]
-            if t.dtype != torch.complex64:
-                raise TypeError(f"{what} {name} has dtype {t.dtype}, the model needs {torch.complex64}")
-            if tuple(t.shape) != (rows, n):
-                raise DimensionMismatch(f"{what} {name} is {tuple(t.shape)}, the model needs {(rows, n)}")
-            if t.device != self.coslat.device:
-                raise ValueError(f"{what} {name} is on {t.device}, the model on {self.coslat.device}")
-            t = t.resolve_conj().contiguous()
+            t = st[name] if name in st else None
+            if not self._plain(t, (rows, n)) or t.dtype != torch.complex64 or t.device != self._dev:
+                return None
+            if not t.is_contiguous() or t.is_conj() or t.is_neg():
+                t = t.resolve_conj().resolve_neg().contiguous()
             keep.append(t)
             ptr.append(t.data_ptr())
         return ptr, keep
 
+    def _check_state(self, st: dict):
+        """Raises for a state that neither form of the equations takes (the transforms convert
+        ln ps from any complex type)."""
+        E, EL, n = self.E, self.E * self.L, self.spectrum.nharm
+        for name, rows in (("vor", EL), ("div", EL), ("temp", EL), ("lnps", E)):
+            t = st[name]
+            if t.dtype != torch.complex64 and name != "lnps":
+                raise TypeError(f"state {name} has dtype {t.dtype}, the model needs {torch.complex64}")
+            if tuple(t.shape) != (rows, n):
+                raise DimensionMismatch(f"state {name} is {tuple(t.shape)}, the model needs {(rows, n)}")
+            if t.device != self._dev:
+                raise ValueError(f"state {name} is on {t.device}, the model on {self._dev}")
+
     def _split(self, x: torch.Tensor) -> dict:
         """The columns vor, div, temp (E*L each) and lnps (E) of one tensor."""
         EL = self.E * self.L
-        vor, div, temp, lnps = x.split((EL, EL, EL, self.E))
+        vor, div, temp, lnps = x.split_with_sizes((EL, EL, EL, self.E))
         return {"vor": vor, "div": div, "temp": temp, "lnps": lnps}
 
     def _vector(self, x: torch.Tensor) -> torch.Tensor:
-        return x.to(device=self.coslat.device, dtype=torch.float32).contiguous()
+        if x.dtype == torch.float32 and x.device == self._dev and x.is_contiguous() and not x.is_neg():
+            return x
+        return x.to(device=self._dev, dtype=torch.float32).resolve_neg().contiguous()
 
     def _model(self):
         """The model's descriptor and the tensors it points to."""
@@ -224,75 +290,163 @@ class DryPrimitiveModel:
         return ShtDryModel(self.L, self.E, self.a, R_DRY, KAPPA, *(t.data_ptr() for t in tables)), tables
 
     def _work(self, with_grid: bool):
-        """The arrays between the kernels of a tendency: spectral columns, grid, grid tendencies."""
-        E, EL, npts, dev = self.E, self.E * self.L, self.grid.npoints, self.coslat.device
+        """The arrays between the kernels of a tendency, as pointers to spectral columns, grid and
+        grid tendencies, and the tensors that hold them: one, or with_grid the grid (as columns)
+        on its own, which then stays."""
+        E, EL, n, npts = self.E, self.E * self.L, self.spectrum.nharm, self.grid.npoints
         down, up = 5 * EL + (3 if with_grid else 2) * E, 6 * EL + E
-        return (torch.empty((max(5 * EL + 3 * E, up), self.spectrum.nharm), dtype=torch.complex64, device=dev),
-                torch.empty((down, npts), device=dev), torch.empty((up, npts), device=dev))
+        spec, fields, g = 2 * n * max(5 * EL + 3 * E, up), npts * up, npts * down
+        spec, fields = (x + -x % 64 for x in (spec, fields))  # 256-byte steps
+        work = torch.empty(spec + fields + (0 if with_grid else g), dtype=torch.float32, device=self._dev)
+        grid = torch.empty((down, npts), dtype=torch.float32, device=self._dev) if with_grid else None
+        p = work.data_ptr()
+        return (p, grid.data_ptr() if with_grid else p + 4 * (spec + fields), p + 4 * spec), (work, grid)
 
     def tendencies(self, st: dict, with_grid: bool = False):
         """Spectral tendencies of vor, div, temp (E*L, nharm) and lnps (E, nharm); with_grid
         also u, v, T (E, L, npoints) and lnps (E, 1, npoints)."""
         L, E = self.L, self.E
-        EL, n, dev = E * L, self.spectrum.nharm, self.coslat.device
-        ptr, keep = self._columns(st, "state")
+        EL, n, dev = E * L, self.spectrum.nharm, self._dev
+        kernels = self._kernels()
+        columns = self._columns(st) if kernels else None
+        if columns is None:
+            if kernels:
+                self._check_state(st)
+            return self._tendencies_arrays(st, with_grid)
+        ptr, keep = columns
         model, tables = self._model()
         tend = torch.empty((3 * EL + E, n), dtype=torch.complex64, device=dev)
-        spec, g, fields = self._work(with_grid)
-        check(lib().sht_dry_tendencies(self.S._plan, C.byref(model), *ptr, tend.data_ptr(), spec.data_ptr(),
-                                       g.data_ptr(), fields.data_ptr(), int(bool(with_grid)), self.S._stream()),
-              "sht_dry_tendencies")
+        work, (held, g) = self._work(with_grid)
+        check(lib().sht_dry_tendencies(self.S._plan, C.byref(model), *ptr, tend.data_ptr(), *work,
+                                       int(bool(with_grid)), self.S._stream()), "sht_dry_tendencies")
         out = self._split(tend)
         if with_grid:
-            o = 2 * EL + 2 * E
-            return out, {"u": g[:EL].view(E, L, -1), "v": g[EL:2 * EL].view(E, L, -1),
-                         "T": g[o:o + EL].view(E, L, -1), "lnps": g[o + 3 * EL:].view(E, 1, -1)}
+            u, v, _, T, _, q = g.split_with_sizes((EL, EL, 2 * E, EL, 2 * EL, E))
+            return out, {"u": u.view(E, L, -1), "v": v.view(E, L, -1), "T": T.view(E, L, -1), "lnps": q.view(E, 1, -1)}
         return out
 
+    def _tendencies_arrays(self, st: dict, with_grid: bool):
+        """The same as array operations around the engine's transforms."""
+        L, E, a = self.L, self.E, self.a
+        ops = self.ops
+        EL = E * L
+        vor, div, temp, lnps = st["vor"], st["div"], st["temp"], st["lnps"]
+        U, V = self.uv(vor, div)
+        g1 = self.synth(torch.cat([U, V, ops.dlambda(lnps), ops.coslat_dlat(lnps)]), unscale=True)
+        g2 = self.synth(torch.cat([temp, div, vor, lnps]))
+        u, v = g1[:EL].view(E, L, -1), g1[EL:2 * EL].view(E, L, -1)
+        dqdx, dqdy = (g1[2 * EL:2 * EL + E] / a).view(E, 1, -1), (g1[2 * EL + E:] / a).view(E, 1, -1)
+        T, D, Z = (g2[i * EL:(i + 1) * EL].view(E, L, -1) for i in range(3))
+        ds, half, full = self.dsigma, self.sigma_half.view(1, -1, 1), self.sigma_full.view(1, -1, 1)
+        uq = u * dqdx + v * dqdy                      # (u, v) . grad ln ps
+        dsum = ds * (D + uq)                          # layer mass-flux divergence
+        csum = torch.cumsum(dsum, dim=1)
+        lnps_t = -csum[:, -1:, :]                     # d ln ps / dt
+        sdot = torch.zeros((E, L + 1, u.shape[-1]), device=self.device)
+        sdot[:, 1:L] = -csum[:, :L - 1] - half[:, 1:L] * lnps_t
+
+        def vadv(X):
+            flux = sdot[:, 1:L] * (X[:, 1:] - X[:, :-1])
+            out = torch.zeros_like(X)
+            out[:, :-1] += flux
+            out[:, 1:] += flux
+            return out / (2 * ds)
+        omp = uq - (csum - 0.5 * dsum) / full         # omega / p on full levels
+        absvor, ci = Z + self.f, self.coslat_inv
+        Au = absvor * v - vadv(u) - R_DRY * T * dqdx
+        Av = -absvor * u - vadv(v) - R_DRY * T * dqdy
+        Tt = T * D - vadv(T) + KAPPA * T * omp
+        flds = ((Au * ci), (Av * ci), (u * T * ci), (v * T * ci), 0.5 * (u * u + v * v), Tt)
+        s = self.analyse(torch.cat([*(x.view(EL, -1) for x in flds), lnps_t.view(E, -1)]))
+        Aus, Avs, uTs, vTs, kes, Tts = (s[i * EL:(i + 1) * EL] for i in range(6))
+        lnps_ts = s[6 * EL:].clone()
+        phi = torch.einsum("kj,ejn->ekn", self.G.to(torch.complex64), temp.view(E, L, -1)).reshape(EL, -1)
+        lnps_ts[:, 0] = 0                              # global mass conservation
+        # the extra degree only serves the vector path: no prognostic tendency there
+        tend = {"vor": ops.curl(Aus, Avs) / a * ops.keep,
+                "div": (ops.divergence(Aus, Avs) / a - ops.laplace(phi + kes) / (a * a)) * ops.keep,
+                "temp": (-ops.divergence(uTs, vTs) / a + Tts) * ops.keep, "lnps": lnps_ts * ops.keep}
+        if with_grid:
+            return tend, {"u": u, "v": v, "T": T, "lnps": g2[3 * EL:].view(E, 1, -1)}
+        return tend
+
     # ------------------------------------------------------------------ time stepping
+    def _diffuse(self, name, x, dt2):
+        nu = self.nu_div if name == "div" else self.nu
+        if name == "lnps":
+            return x
+        return x / (1.0 + dt2 * nu)
+
+    def _step_kernels(self, tend):
+        """_columns of the state, of the previous one and of the tendencies (None: none) where
+        the time-step kernels state the step; otherwise None."""
+        n, now, prev = (self.spectrum.nharm,), self.state, self.state_prev
+        if not (self._untraced() and type(self)._diffuse is _DIFFUSE and "_diffuse" not in vars(self)
+                and isinstance(self.dt, (int, float)) and isinstance(self.robert, (int, float))
+                and isinstance(self.williams, (int, float)) and self._plain(self.nu, n) and self._plain(self.nu_div, n)
+                and not self.nu.is_complex() and not self.nu_div.is_complex() and len(now) == 4):
+            return None
+        columns = [None if st is None else self._columns(st) for st in (now, prev, tend)]
+        if any(c is None and st is not None for c, st in zip(columns, (now, prev, tend))):
+            return None
+        return columns
+
     def step(self, correction=None):
         """One leapfrog step (Euler forward for the first); `correction(model, tend, grid)`
         may add to the spectral tendencies."""
         # without a correction the tendencies go straight into the step, unless a subclass or an
         # instance has its own, or the class was given another
-        fused = correction is None and "tendencies" not in vars(self) and type(self).tendencies is _TENDENCIES
-        L, E, n, dev = self.L, self.E, self.spectrum.nharm, self.coslat.device
-        rows = 3 * E * L + E
-        if not fused:
+        fused = (correction is None and "tendencies" not in vars(self) and type(self).tendencies is _TENDENCIES
+                 and self._kernels())
+        columns = self._step_kernels(None) if fused else None
+        if columns is None:
             need_grid = correction is not None
             out = self.tendencies(self.state, with_grid=need_grid)
             tend, grid = (out if need_grid else (out, None))
             if correction is not None:
                 correction(self, tend, grid)
-            tptr, tkeep = self._columns(tend, "tendency")
+            columns = self._step_kernels(tend)
+        dt2 = self.dt if self.state_prev is None else 2.0 * self.dt
+        w1 = self.robert * self.williams / 2
+        w2 = self.robert * (1 - self.williams) / 2
+        if columns is not None:
+            filtered, new = self._leapfrog(*columns, dt2, w1, w2)
+        else:
+            base = self.state if self.state_prev is None else self.state_prev
+            new = {k: self._diffuse(k, base[k] + dt2 * tend[k], dt2) for k in self.state}
+            filtered = {}
+            if self.state_prev is not None:
+                for k in self.state:
+                    d = self.state_prev[k] - 2 * self.state[k] + new[k]
+                    filtered[k] = self.state[k] + w1 * d
+                    new[k] = new[k] - w2 * d
+        self.state_prev, self.state = {**self.state, **filtered}, new
+        self.nsteps += 1
+
+    def _leapfrog(self, now, prev, tend, dt2, w1, w2):
+        """The filtered present state and the next one from _columns of the present state, of the
+        previous one (None: the first step) and of the tendencies (None: the state's own)."""
+        L, E, n, dev = self.L, self.E, self.spectrum.nharm, self._dev
+        nu, nu_div = self._vector(self.nu), self._vector(self.nu_div)
+        arr = C.c_void_p * 4
+        new = torch.empty((3 * E * L + E, n), dtype=torch.complex64, device=dev)
+        state, filtered = arr(*now[0]), None
+        if prev is not None:
+            filtered, prev = torch.empty_like(new), arr(*prev[0])
+        out = (None if filtered is None else filtered.data_ptr(), new.data_ptr())
+        if tend is None:
+            model, tables = self._model()
+            work, held = self._work(False)
+            check(lib().sht_dry_step(self.S._plan, C.byref(model), state, prev, nu.data_ptr(), nu_div.data_ptr(),
+                                     dt2, w1, w2, *out, *work, self.S._stream()), "sht_dry_step")
+        else:
+            tptr, tkeep = tend
             if any(p != tptr[0] + 8 * n * E * L * i for i, p in enumerate(tptr)):  # a correction put its own tensors there
                 tkeep = torch.cat(tkeep)
                 tptr = [tkeep.data_ptr()]
-        sptr, skeep = self._columns(self.state, "state")
-        nu, nu_div = self._vector(self.nu), self._vector(self.nu_div)
-        arr = C.c_void_p * 4
-        new = torch.empty((rows, n), dtype=torch.complex64, device=dev)
-        if self.state_prev is None:
-            dt2, prev, filtered = self.dt, None, None
-        else:
-            pptr, pkeep = self._columns(self.state_prev, "previous state")
-            filtered = torch.empty_like(new)
-            dt2, prev = 2.0 * self.dt, arr(*pptr)
-        w1 = self.robert * self.williams / 2
-        w2 = self.robert * (1 - self.williams) / 2
-        out = (None if filtered is None else filtered.data_ptr(), new.data_ptr())
-        if fused:
-            model, tables = self._model()
-            spec, g, fields = self._work(False)
-            check(lib().sht_dry_step(self.S._plan, C.byref(model), arr(*sptr), prev, nu.data_ptr(), nu_div.data_ptr(),
-                                     dt2, w1, w2, *out, spec.data_ptr(), g.data_ptr(), fields.data_ptr(),
-                                     self.S._stream()), "sht_dry_step")
-        else:
-            check(lib().sht_dry_leapfrog(self.S._plan, L, E, arr(*sptr), prev, tptr[0], nu.data_ptr(),
+            check(lib().sht_dry_leapfrog(self.S._plan, L, E, state, prev, tptr[0], nu.data_ptr(),
                                          nu_div.data_ptr(), dt2, w1, w2, *out, self.S._stream()), "sht_dry_leapfrog")
-        self.state_prev = self.state if filtered is None else self._split(filtered)
-        self.state = self._split(new)
-        self.nsteps += 1
+        return {} if filtered is None else self._split(filtered), self._split(new)
 
     # ------------------------------------------------------------------ initial conditions
     def jet_state(self, seeds, u0=35.0, lat0=30.0, width=10.0, T0=288.0, lapse=0.0065,
@@ -343,4 +497,10 @@ class DryPrimitiveModel:
         self.S.close()
 
 
-_TENDENCIES = DryPrimitiveModel.tendencies  # what step() may fuse with the time step
+# The methods and operators that the kernels stand for, and the tensors that are plain memory.
+_TENDENCIES, _DIFFUSE = DryPrimitiveModel.tendencies, DryPrimitiveModel._diffuse
+_METHODS = {"_lta", "synth", "analyse", "uv", "_tendencies_arrays"}
+_methods = operator.attrgetter(*_METHODS)
+_operators = operator.attrgetter("dlambda", "coslat_dlat", "divergence", "curl", "laplace")
+_METHODS_AS_BUILT, _OPERATORS_AS_BUILT = _methods(DryPrimitiveModel), _operators(SpectralOps)
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
