@@ -274,9 +274,10 @@ class DryPrimitiveModel:
                 raise ValueError(f"state {name} is on {t.device}, the model on {self._dev}")
 
     def _split(self, x: torch.Tensor) -> dict:
-        """The columns vor, div, temp (E*L each) and lnps (E) of one tensor."""
+        """The columns vor, div, temp (E*L each) and lnps (E) of one tensor, each a tensor of
+        its own to autograd (no view of the others)."""
         EL = self.E * self.L
-        vor, div, temp, lnps = x.split_with_sizes((EL, EL, EL, self.E))
+        vor, div, temp, lnps = x.unsafe_split_with_sizes((EL, EL, EL, self.E))
         return {"vor": vor, "div": div, "temp": temp, "lnps": lnps}
 
     def _vector(self, x: torch.Tensor) -> torch.Tensor:
@@ -321,7 +322,7 @@ class DryPrimitiveModel:
                                        int(bool(with_grid)), self.S._stream()), "sht_dry_tendencies")
         out = self._split(tend)
         if with_grid:
-            u, v, _, T, _, q = g.split_with_sizes((EL, EL, 2 * E, EL, 2 * EL, E))
+            u, v, _, T, _, q = g.unsafe_split_with_sizes((EL, EL, 2 * E, EL, 2 * EL, E))
             return out, {"u": u.view(E, L, -1), "v": v.view(E, L, -1), "T": T.view(E, L, -1), "lnps": q.view(E, 1, -1)}
         return out
 
