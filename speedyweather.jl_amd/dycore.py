@@ -421,7 +421,9 @@ class DryPrimitiveModel:
                     d = self.state_prev[k] - 2 * self.state[k] + new[k]
                     filtered[k] = self.state[k] + w1 * d
                     new[k] = new[k] - w2 * d
-        self.state_prev, self.state = {**self.state, **filtered}, new
+        for k in filtered:
+            self.state[k] = filtered[k]
+        self.state_prev, self.state = self.state, new
         self.nsteps += 1
 
     def _leapfrog(self, now, prev, tend, dt2, w1, w2):

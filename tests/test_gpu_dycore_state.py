@@ -27,3 +27,15 @@ def test_tendencies_are_changed_in_place_one_by_one(sw, gpu):
         m.state["temp"] = m.state["temp"].detach()
         m.state["vor"] *= 1.0 + 0j
     m.close()
+
+
+def test_a_held_state_becomes_the_filtered_one(sw, gpu):
+    """The filter writes the present state's dictionary, which then is the previous one."""
+    m = sw.dycore.DryPrimitiveModel(21, 8)
+    m.set_state(state(sw, m, 10))
+    m.step()
+    held, before = m.state, dict(m.state)
+    m.step()
+    assert m.state_prev is held
+    assert not torch.equal(held["vor"], before["vor"])
+    m.close()
