@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void dry_grid_kernel(const float *__restrict__
     const int L = LT ? LT : Lrt;
     const long long np = npoints, EL = (long long)E * L;
     const float ci = as_global(coslat_inv_)[p], f = as_global(coriolis_)[p];
-    const float ds = 1.f / (float)L, h = 1.f / (2.f * ds);
+    const float ds = 1.f / (float)L, h = 0.5f * (float)L;  // layer thickness; 1 / (2 ds), exactly
     for (int e = blockIdx.y; e < E; e += gridDim.y) {
         const SHT_GLOBAL float *g = as_global(g_) + p;
         const SHT_GLOBAL float *gq = g + 2 * EL * np;
@@ -162,7 +162,8 @@ __device__ __forceinline__ void dry_step(float2 x, float2 b, float2 t, float dam
 
 // Spectral tendencies (columns: vorticity, divergence, temperature EL each, ln ps E) from the
 // analysed fields s (columns of dry_grid_kernel) and the temperature (geopotential, G L x L
-// with zeros below the diagonal).  One thread per coefficient and level.  LT levels known at
+// with zeros below the diagonal); ri, rr: the radius's reciprocal and its square's, rounded from
+// 64 bits as the array operations round them.  One thread per coefficient and level.  LT levels known at
 // compile time: the temperatures of the levels below are all in flight at once (8 members and
 // levels: T31 5.2 -> 3.8 us, T127 13.6 -> 12.7); LT = 0: L levels, one load after another.
 // STEP: the tendencies are not stored but applied (dry_step), one pass over the state instead of
@@ -171,7 +172,7 @@ template <int LT, bool STEP>
 __global__ __launch_bounds__(256) void dry_tendency_kernel(const DevPlan *__restrict__ PP, const float2 *__restrict__ s_,
                                                            const float2 *__restrict__ temp_,
                                                            const float *__restrict__ G_, float2 *__restrict__ tend_,
-                                                           int Lrt, int E, float radius, float radius2, DryStep S) {
+                                                           int Lrt, int E, float ri, float rr, DryStep S) {
 #pragma clang fp contract(off)
     const int L = LT > 0 ? LT : Lrt;
     const DevPlan &P = *PP;
@@ -248,7 +249,6 @@ __global__ __launch_bounds__(256) void dry_tendency_kernel(const DevPlan *__rest
             }
         }
         const float2 iu = cneg_i(mx, u), iv = cneg_i(mx, v), iuT = cneg_i(mx, uT);
-        const float ri = 1.f / radius, rr = 1.f / radius2;
         const float2 curl = make_float2(iv.x + gy.x * um.x - gy.y * up.x, iv.y + gy.x * um.y - gy.y * up.y);
         const float2 div = make_float2(iu.x - gy.x * vm.x + gy.y * vp.x, iu.y - gy.x * vm.y + gy.y * vp.y);
         const float2 divT = make_float2(iuT.x - gy.x * vTm.x + gy.y * vTp.x, iuT.y - gy.x * vTm.y + gy.y * vTp.y);
@@ -310,7 +310,7 @@ static int launch_tendency(const DevPlan *P, int nharm, const void *s, const flo
     const dim3 grid((nharm + 255) / 256, std::min(E * L + E, kMaxGridY));
     auto *f = L == 8 ? &dry_tendency_kernel<8, STEP> : &dry_tendency_kernel<0, STEP>;
     f<<<grid, 256, 0, as_stream(stream)>>>(P, static_cast<const float2 *>(s), temp, G, static_cast<float2 *>(tend), L, E,
-                                           (float)radius, (float)(radius * radius), S);
+                                           (float)(1.0 / radius), (float)(1.0 / (radius * radius)), S);
     return (int)hipGetLastError();
 }
 

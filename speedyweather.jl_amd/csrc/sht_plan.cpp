@@ -1668,7 +1668,7 @@ static int dry_tendencies(sht_plan *plan, const sht_dry_model *model, const sht:
     rc = run_synthesis(plan, spec, nharm, grid, np, down, 0, 0, 0, stream, LapOp(), nullptr, 2 * E * L + 2 * E);
     if (rc) return rc;
     rc = launched(sht::launch_dry_grid(static_cast<const float *>(grid), static_cast<float *>(fields), model->coslat_inv,
-                                       model->coriolis, np, L, E, 1.f / (float)model->radius, (float)model->r_dry,
+                                       model->coriolis, np, L, E, (float)(1.0 / model->radius), (float)model->r_dry,
                                        (float)model->kappa, stream),
                   "dry grid tendencies");
     if (rc) return rc;
