@@ -41,8 +41,6 @@ class _RingGrid:
         if nlat_half < 1:
             raise ValueError("nlat_half must be >= 1")
         self.nlat_half = int(nlat_half)
-        # every transform call compares sizes with it
-        self.npoints = 2 * sum(self.nlon_ring(j) for j in range(self.nlat_half))
 
     def nlon_ring(self, j: int) -> int:  # 0-based northern ring
         raise NotImplementedError
@@ -55,6 +53,10 @@ class _RingGrid:
     def nlons(self) -> np.ndarray:
         north = [self.nlon_ring(j) for j in range(self.nlat_half)]
         return np.array(north + north[::-1])
+
+    @property
+    def npoints(self) -> int:
+        return int(self.nlons.sum())
 
     @property
     def nlon_max(self) -> int:
@@ -79,6 +81,10 @@ class OctahedralGaussianGrid(_RingGrid):
     def nlon_ring(self, j: int) -> int:
         return 16 + 4 * (j + 1)
 
+    @property
+    def npoints(self) -> int:  # the sum, in closed form: every transform call compares sizes with it
+        return 4 * self.nlat_half * (self.nlat_half + 9)
+
 
 class FullGaussianGrid(_RingGrid):
     """4 nlat_half points on every ring."""
@@ -86,6 +92,10 @@ class FullGaussianGrid(_RingGrid):
 
     def nlon_ring(self, j: int) -> int:
         return 4 * self.nlat_half
+
+    @property
+    def npoints(self) -> int:
+        return 8 * self.nlat_half * self.nlat_half
 
 
 class Field:

@@ -18,13 +18,16 @@ class Spectrum:
         if not (1 <= mmax <= lmax):
             raise ValueError("need 1 <= mmax <= lmax")
         self.lmax, self.mmax = int(lmax), int(mmax)
-        # nonzeros (spectrum.jl:87-89); every transform call compares sizes with it
-        self.nharm = self.lmax * self.mmax - self.mmax * (self.mmax - 1) // 2
 
     @classmethod
     def from_truncation(cls, truncation: int, one_more_degree: bool = False) -> "Spectrum":
         """Spectrum(truncation; one_degree_more) (spectrum.jl:72-78)."""
         return cls(truncation + int(one_more_degree), truncation)
+
+    @property
+    def nharm(self) -> int:
+        """nonzeros (spectrum.jl:87-89)."""
+        return self.lmax * self.mmax - self.mmax * (self.mmax - 1) // 2
 
     def offset(self, m: int) -> int:
         """0-based packed start of order m (0-based)."""
