@@ -171,17 +171,25 @@ __device__ __forceinline__ void put_f(u16 *lds, int f, int n, unsigned a, unsign
     *reinterpret_cast<unsigned *>(lds + o) = __builtin_amdgcn_perm(dpp_xor1(a), a, sel);
     *reinterpret_cast<unsigned *>(lds + o + 2 * kSF) = __builtin_amdgcn_perm(dpp_xor1(b), b, sel);
 }
-// BF16 parts of four FP32 values as packed pairs: part[q][0..1], hi + mid + lo = v exactly.
+// BF16 parts of four FP32 values as packed pairs: part[q][0..1], hi + mid + lo = v exactly.  hi
+// is truncated, not rounded, and the rest of an infinity is 0, so that products of the parts
+// overflow only where those of v do (rounded up, hi may exceed the range that v is in; inf - inf
+// would make the rest NaN).
+__device__ __forceinline__ float nan_to_zero(float r) {
+    float z;  // the median of r, r, 0; with a NaN among them the least number
+    asm("v_med3_f32 %0, %1, %1, 0" : "=v"(z) : "v"(r));
+    return z;
+}
 __device__ __forceinline__ void split4(const float (&v)[4], unsigned (&part)[3][2]) {
-    float r[4] = {v[0], v[1], v[2], v[3]};
+    float r[4];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
+    for (int e = 0; e < 4; ++e) r[e] = nan_to_zero(v[e] - __uint_as_float(__float_as_uint(v[e]) & 0xFFFF0000u));
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            part[q][k] = pack_bf16(r[2 * k], r[2 * k + 1]);
-            r[2 * k] -= __uint_as_float(part[q][k] << 16);
-            r[2 * k + 1] -= __uint_as_float(part[q][k] & 0xFFFF0000u);
-        }
+    for (int k = 0; k < 2; ++k) {
+        part[0][k] = __builtin_amdgcn_perm(__float_as_uint(v[2 * k + 1]), __float_as_uint(v[2 * k]), 0x07060302u);
+        part[1][k] = pack_bf16(r[2 * k], r[2 * k + 1]);
+        part[2][k] = pack_bf16(r[2 * k] - __uint_as_float(part[1][k] << 16),
+                               r[2 * k + 1] - __uint_as_float(part[1][k] & 0xFFFF0000u));
     }
 }
 __device__ __forceinline__ bf16x8 frag_n(const u16 *lds, int n, int pos) {
