@@ -275,9 +275,16 @@ int sht_mlp_create(int32_t device, int32_t max_batch, sht_mlp **mlp);
 int sht_mlp_set_params(sht_mlp *mlp, const float *host_params);
 int sht_mlp_get_params(sht_mlp *mlp, float *host_params);
 int sht_mlp_forward(sht_mlp *mlp, const float *x, float *y, int32_t B, void *stream);
-/* gradient of the loss w.r.t. the parameters (no update) and the loss */
+/* gradient of the loss w.r.t. the parameters (no update) and the loss; partial sums go through
+ * the handle's scratch, so gradients and training steps of one handle belong on one stream (from
+ * any threads) or must be ordered among themselves */
 int sht_mlp_gradient(sht_mlp *mlp, const float *x, const float *t, int32_t B, float *grad, float *loss,
                      void *stream);
+/* the same through a scratch of the caller's, at least sht_mlp_scratch_bytes(B) bytes of device
+ * memory: gradients with scratches of their own may overlap, as forward calls may */
+int64_t sht_mlp_scratch_bytes(int32_t B);
+int sht_mlp_gradient_scratch(sht_mlp *mlp, const float *x, const float *t, int32_t B, float *grad, float *loss,
+                             void *scratch, void *stream);
 /* one Adam step (beta 0.9 / 0.999, eps 1e-8) with learning rate lr; loss may be null */
 int sht_mlp_train_step(sht_mlp *mlp, const float *x, const float *t, int32_t B, float lr, float *loss,
                        void *stream);

@@ -31,7 +31,7 @@ EXPORTS = (
     "sht_grid2spec_pullback", "sht_divergence", "sht_laplace", "sht_gradient", "sht_plan_create_matrix",
     "sht_synthesis_laplace", "sht_analysis_laplace", "sht_time_stage", "sht_tune_cache_save",
     "sht_tune_cache_load", "sht_transform_static", "sht_plan_set_graphs", "sht_plan_graph_count",
-    "sht_dry_tendencies", "sht_dry_leapfrog", "sht_dry_step",
+    "sht_dry_tendencies", "sht_dry_leapfrog", "sht_dry_step", "sht_mlp_scratch_bytes", "sht_mlp_gradient_scratch",
 )
 
 
@@ -114,6 +114,8 @@ def lib() -> C.CDLL:
         L.sht_mlp_get_params.argtypes = [vp, vp]
         L.sht_mlp_forward.argtypes = [vp, vp, vp, i32, vp]
         L.sht_mlp_gradient.argtypes = [vp, vp, vp, i32, vp, vp, vp]
+        L.sht_mlp_scratch_bytes.argtypes, L.sht_mlp_scratch_bytes.restype = [i32], C.c_int64
+        L.sht_mlp_gradient_scratch.argtypes = [vp, vp, vp, i32, vp, vp, vp, vp]
         L.sht_mlp_train_step.argtypes = [vp, vp, vp, i32, C.c_float, vp, vp]
         L.sht_mlp_destroy.argtypes = [vp]
         L.sht_plan_autotune.argtypes = [vp, i32, vp]

@@ -16,6 +16,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -491,6 +492,7 @@ struct sht_mlp {
     float *P = nullptr, *M = nullptr, *V = nullptr, *Gp = nullptr, *Lp = nullptr, *loss = nullptr;
     bf16 *Wf = nullptr;  // BF16 weights in fragment order
     long long step = 0;
+    std::mutex launch;
 };
 
 namespace {
@@ -591,17 +593,18 @@ int sht_mlp_forward(sht_mlp *m, const float *x, float *y, int32_t B, void *strea
     return e == hipSuccess ? SHT_OK : mlp_fail(SHT_ERR_HIP, hipGetErrorString(e));
 }
 
-// Partial gradients of the loss, then their sum into grad (adam null) or an Adam step.
+// Partial gradients and losses (into Gp, Lp), then their sum into grad (adam null) or an Adam step.
 static int mlp_grad(sht_mlp *m, const float *x, const float *t, int B, float *grad, float *loss,
-                    const AdamArgs *adam, void *stream) {
+                    const AdamArgs *adam, float *Gp, float *Lp, void *stream) {
     int tiles = 0;
     const int nblk = grad_blocks(B, tiles);
-    mlp_gradient_kernel<<<nblk, kGradThreads, kGradLds, st(stream)>>>(m->Wf, m->P, x, t, m->Gp, m->Lp, B, tiles);
+    std::lock_guard<std::mutex> lock(m->launch);  // another thread's pair may use the same partials
+    mlp_gradient_kernel<<<nblk, kGradThreads, kGradLds, st(stream)>>>(m->Wf, m->P, x, t, Gp, Lp, B, tiles);
     const int rblk = (kMlpParams + 63) / 64;
     if (adam)
-        mlp_reduce_kernel<true><<<rblk, 256, 0, st(stream)>>>(m->Gp, nullptr, m->Lp, loss, nblk, B, *adam);
+        mlp_reduce_kernel<true><<<rblk, 256, 0, st(stream)>>>(Gp, nullptr, Lp, loss, nblk, B, *adam);
     else
-        mlp_reduce_kernel<false><<<rblk, 256, 0, st(stream)>>>(m->Gp, grad, m->Lp, loss, nblk, B, AdamArgs{});
+        mlp_reduce_kernel<false><<<rblk, 256, 0, st(stream)>>>(Gp, grad, Lp, loss, nblk, B, AdamArgs{});
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? SHT_OK : mlp_fail(SHT_ERR_HIP, hipGetErrorString(e));
 }
@@ -609,7 +612,22 @@ static int mlp_grad(sht_mlp *m, const float *x, const float *t, int B, float *gr
 int sht_mlp_gradient(sht_mlp *m, const float *x, const float *t, int32_t B, float *grad, float *loss, void *stream) {
     if (!m || !x || !t || !grad || !loss || B < 1 || B > m->max_batch) return mlp_fail(SHT_ERR_ARG, "bad arguments");
     Dev g(m->device);
-    return mlp_grad(m, x, t, B, grad, loss, nullptr, stream);
+    return mlp_grad(m, x, t, B, grad, loss, nullptr, m->Gp, m->Lp, stream);
+}
+
+int64_t sht_mlp_scratch_bytes(int32_t B) {
+    int tiles = 0;
+    return B < 1 ? 0 : (int64_t)grad_blocks(B, tiles) * (kMlpParams + 1) * 4;
+}
+
+int sht_mlp_gradient_scratch(sht_mlp *m, const float *x, const float *t, int32_t B, float *grad, float *loss,
+                             void *scratch, void *stream) {
+    if (!m || !x || !t || !grad || !loss || !scratch || B < 1 || B > m->max_batch)
+        return mlp_fail(SHT_ERR_ARG, "bad arguments");
+    Dev g(m->device);
+    int tiles = 0;
+    float *Gp = static_cast<float *>(scratch);
+    return mlp_grad(m, x, t, B, grad, loss, nullptr, Gp, Gp + (size_t)grad_blocks(B, tiles) * kMlpParams, stream);
 }
 
 int sht_mlp_train_step(sht_mlp *m, const float *x, const float *t, int32_t B, float lr, float *loss, void *stream) {
@@ -619,7 +637,7 @@ int sht_mlp_train_step(sht_mlp *m, const float *x, const float *t, int32_t B, fl
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.f - powf(b1, (float)m->step), c2 = 1.f - powf(b2, (float)m->step);
     const AdamArgs adam{m->P, m->Wf, m->M, m->V, lr, b1, b2, 1e-8f, c1, c2};
-    const int rc = mlp_grad(m, x, t, B, nullptr, loss ? loss : m->loss, &adam, stream);
+    const int rc = mlp_grad(m, x, t, B, nullptr, loss ? loss : m->loss, &adam, m->Gp, m->Lp, stream);
     if (rc) m->step -= 1;
     return rc;
 }
