@@ -554,19 +554,20 @@ __device__ __forceinline__ FFTPass load_pass(const SHT_GLOBAL FFTPass *p) {
     d.l = q[1];
     d.M = q[2];
     d.mulM = (unsigned)q[3];
-    d.mulR = (unsigned)q[4];
     return d;
 }
 
-// Runs all passes in place on buf (kFFTCols columns of N points, the first ncol of them
-// data): a first-pass MFMA radix, then the register passes (pd: the first one's descriptor), all across the workgroup.  Every pass ends with a barrier.
-// The plan tables the FFT kernels read, fetched with the ring record (one level of scalar
-// loads), and the first register pass's descriptor, fetched before the ring's data.
+// The plan tables the FFT kernels read, fetched with the ring record (one level of scalar loads).
 struct FFTPlanTables {
     const float *twiddle;
     const FFTPass *passes;
     const unsigned short *prime_tab;
 };
+
+// Runs all passes in place on buf (kFFTCols columns of N points, the first ncol of them data):
+// a first-pass MFMA radix, then the register passes, all across the workgroup.  pd: the first
+// register pass's descriptor, fetched before the ring's data.  Every pass ends with a barrier,
+// but LAST's, which stores the grid.
 
 template <bool INV, bool LAST, int MAXN>
 __device__ __attribute__((always_inline)) void fft_run(const FFTPlanTables &P, const FFTRing &R, float2 *buf,
@@ -581,7 +582,6 @@ __device__ __attribute__((always_inline)) void fft_run(const FFTPlanTables &P, c
         p0.l = 1;
         p0.M = R.M0;
         p0.mulM = R.mulM0;
-        p0.mulR = R.mulR0;
         const SHT_GLOBAL b8 *tab = reinterpret_cast<const SHT_GLOBAL b8 *>(as_global(P.prime_tab)) + R.prime_off;
         const int h = (p0.R - 1) >> 1;
         const int tmax = INV ? min(h, (mt + p0.M - 1) / p0.M) : h;
@@ -639,7 +639,6 @@ __device__ __forceinline__ FFTRing load_ring(const SHT_GLOBAL FFTRing *p) {
     r.prime = q[5];
     r.M0 = q[6];
     r.mulM0 = (unsigned)q[7];
-    r.mulR0 = (unsigned)q[8];
     r.tw_off = w[6];
     r.fboff = w[7];
     r.ring_n = w[8];

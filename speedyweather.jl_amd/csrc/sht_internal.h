@@ -190,29 +190,28 @@ __host__ __device__ inline int dft_smem_bytes(bool synthesis, bool f16, int cg, 
 }
 
 // One pass of a ring FFT (radix R, l = product of the earlier radices, M = N / (l R)) with
-// the multipliers of FastDiv for M and R precomputed, so the kernels divide by neither.
+// the multiplier of FastDiv for M precomputed, so the kernels do not divide by it.
 struct FFTPass {
     int R, l, M;
-    unsigned mulM, mulR;
-    int pad[3];
+    unsigned mulM;
 };
 // FastDiv multiplier of d: x / d == umulhi(x, mul) for x, d < 2^16.
 inline unsigned fastdiv_mul(int d) { return d > 1 ? 0xFFFFFFFFu / (unsigned)d + 1u : 0u; }
 
 // One FFT workgroup rank's ring (launch order, heaviest first, per factorisation policy):
 // everything the FFT kernels read per ring in one record, so that a workgroup's first loads
-// depend on no other load.  prime, M0, mulM0, mulR0: the MFMA first pass (radix, butterflies
-// per column, FastDiv multipliers of M0 and prime), prime = 0 without one.
+// depend on no other load.  prime, M0, mulM0: the MFMA first pass (radix, butterflies
+// per column, FastDiv multiplier of M0), prime = 0 without one.
 struct FFTRing {
     int j, N, mt, mte;
     int nf, prime, M0;
-    unsigned mulM0, mulR0;
-    int pad[3];
+    unsigned mulM0;
+    int pad[4];
     long long tw_off;     // first twiddle of the ring
     long long fboff;      // first Fourier-buffer row
     long long ring_n;     // first grid point of the northern ring
     long long ring_s;     // first grid point of the southern ring
-    long long prime_off;  // the MFMA first pass's table (DevPlan::prime_tab, 8-element vectors)
+    long long prime_off;  // the MFMA first pass's table (DevPlan::prime_tab, vectors of 8)
     long long passes;     // first pass descriptor (index into DevPlan::passes)
 };
 static_assert(sizeof(FFTRing) == 96, "FFTRing layout");
@@ -240,15 +239,7 @@ struct DevPlan {
     const int *ring_order;    // FFT workgroup -> ring, most expensive first
     const FFTRing *rings;     // FFT workgroup rank -> its ring's record (same order)
 
-    // per order m
-    const int *j0;               // first ring with mt >= m (rings j0..n-1 contribute)
-    const long long *lm_off;     // packed offset of column m
-    const long long *syn_off;    // offset of m's block in the synthesis Λ arrays
-    const long long *ana_off;    // offset of m's block in the analysis Λ arrays
-    const long long *syn_soff;   // offset of m's row scales (synthesis, per ring)
-    const long long *ana_soff;   // offset of m's row scales (analysis, per degree)
-
-    // Λ in MFMA-fragment order.  FP32 mode: float arrays.  Split modes: arrays of 16-bit
+    // Λ in MFMA-fragment order (an order's offsets come with its tiles: LegTile).  FP32 mode: float arrays.  Split modes: arrays of 16-bit
     // parts, v = hi + lo (scaled FP16) or v = hi + mid + lo (BF16, three terms), and
     // inverse row scales (FP16 only).
     const float *syn_f32;
@@ -266,13 +257,12 @@ struct DevPlan {
     const float *twiddle;  // interleaved complex exp(-2 pi i k / N) for each ring
     const long long *tw_off;
     const FFTPass *passes;  // kMaxFactors passes per ring, in order
-    const int *nfac;
     // First-pass prime radices r (MFMA pass): per r, cos / sin(2 pi s t / r) for rows
     // s = 0..h (tiles of 16) and t = 1..h (chunks of 32), h = (r-1)/2, as three BF16 parts of
     // the FP64 values in MFMA fragment order: per (row tile, chunk) six fragments (cos hi, mid,
-    // lo, sin hi, mid, lo) of a vector of 8 per lane, 1 KiB contiguous each.  prime_off[r] (r < 256): r's first vector.
+    // lo, sin hi, mid, lo) of a vector of 8 per lane, 1 KiB contiguous each (FFTRing::prime_off:
+    // a ring's first vector).
     const unsigned short *prime_tab;
-    const long long *prime_off;
     // Ring DFT on MFMA (rings of N = 4p points): per ring, the cos / sin matrices
     // cos(2 pi r t / p), sin(2 pi r t / p), rows r = 0..p/2 (tiles of 16), columns
     // t = 1..(p-1)/2, in MFMA fragment order: FP32 (dft32, chunks of 16 t, a float4 of cos

@@ -543,12 +543,12 @@ int factorize(int N, int *fac, const FFTPolicy &pol) {
 
 // Per-ring pass descriptors of a factorisation (radix, l, M and their division multipliers).
 std::vector<sht::FFTPass> pass_table(const Geometry &g, const std::vector<int> &fac, const std::vector<int> &nfac) {
-    std::vector<sht::FFTPass> t((size_t)g.n * sht::kMaxFactors, sht::FFTPass{1, 1, 1, 0u, 0u, {0, 0, 0}});
+    std::vector<sht::FFTPass> t((size_t)g.n * sht::kMaxFactors, sht::FFTPass{1, 1, 1, 0u});
     for (int j = 0; j < g.n; ++j) {
         int l = 1;
         for (int f = 0; f < nfac[j]; ++f) {
             const int R = fac[(size_t)j * sht::kMaxFactors + f], M = g.nlon[j] / (l * R);
-            t[(size_t)j * sht::kMaxFactors + f] = sht::FFTPass{R, l, M, sht::fastdiv_mul(M), sht::fastdiv_mul(R), {0, 0, 0}};
+            t[(size_t)j * sht::kMaxFactors + f] = sht::FFTPass{R, l, M, sht::fastdiv_mul(M)};
             l *= R;
         }
     }
@@ -939,12 +939,6 @@ int build_plan(sht_plan *pl) {
     if ((rc = dev_upload(A, coslat_f, &P.coslat_inv))) return rc;
     std::vector<float> domega_f(dOmega.begin(), dOmega.end());
     if ((rc = dev_upload(A, domega_f, &P.domega))) return rc;
-    if ((rc = dev_upload(A, g.j0, &P.j0))) return rc;
-    if ((rc = dev_upload(A, g.lm_off, &P.lm_off))) return rc;
-    if ((rc = dev_upload(A, syn_off, &P.syn_off))) return rc;
-    if ((rc = dev_upload(A, ana_off, &P.ana_off))) return rc;
-    if ((rc = dev_upload(A, syn_soff, &P.syn_soff))) return rc;
-    if ((rc = dev_upload(A, ana_soff, &P.ana_soff))) return rc;
     if (split) {
         const uint16_t *p16;
         if ((rc = dev_upload(A, syn_hi, &p16))) return rc;
@@ -973,7 +967,6 @@ int build_plan(sht_plan *pl) {
         std::vector<uint16_t> ptab;
         prime_tables(fac_v, nfac_v, pl->pol_ok, n, ptab, poff);
         if ((rc = dev_upload(A, ptab, &P.prime_tab))) return rc;
-        if ((rc = dev_upload(A, poff, &P.prime_off))) return rc;
     }
     if ((rc = dev_upload(A, tw_off, &P.tw_off))) return rc;
     {
@@ -1082,7 +1075,6 @@ int build_plan(sht_plan *pl) {
                     x.prime = R0;
                     x.M0 = x.N / R0;
                     x.mulM0 = sht::fastdiv_mul(x.M0);
-                    x.mulR0 = sht::fastdiv_mul(R0);
                     x.prime_off = poff[R0];
                 }
                 x.tw_off = tw_off[j];
@@ -1097,7 +1089,6 @@ int build_plan(sht_plan *pl) {
             }
             if ((rc = dev_upload(A, rings, &views[q].rings))) return rc;
             if ((rc = dev_upload(A, pass_table(g, fac_v[q], nfac_v[q]), &views[q].passes))) return rc;
-            if ((rc = dev_upload(A, nfac_v[q], &views[q].nfac))) return rc;
             pl->Pv[q] = views[q];
         }
         if ((rc = dev_upload(A, views, &pl->dPv))) return rc;

@@ -271,14 +271,14 @@ DenseSplit dense_split(long long M, long long N, int K) {
     // split: shorter ones spend their time on partial sums (T31 K=32, round trip: 21.7 us with
     // 16 groups, 43.8 with 2; T63 K=32: 106.7 us with 1024 workgroups, 110.5 with 2048, 118.1
     // with 3072).
-    auto splits = [&](long long want, int &per) {  // of at least `want` equal parts, none empty
+    auto splits = [&](long long want, int &per) {  // of at most `want` equal parts, none empty
         want = std::max(1LL, std::min(want, d.s4));
         per = (int)((d.s4 + want - 1) / want);
         return (int)((d.s4 + per - 1) / per);
     };
     d.s = splits(std::min((1024 + wgs - 1) / wgs, d.s4 / kDenseMinGroups), d.s4_split);
     int per;
-    d.s_work = splits((2048 + wgs - 1) / wgs, per);  // callers' scratch limits count on this size
+    d.s_work = splits((2048 + wgs - 1) / wgs, per);  // plans are accepted and refused by this size
     return d;
 }
 
