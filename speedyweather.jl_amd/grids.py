@@ -3,6 +3,7 @@ full_gaussian.jl:17-61, field.jl:7-18) and the resolution rules of
 SpeedyTransforms/src/aliasing.jl:9-69."""
 from __future__ import annotations
 
+import functools
 import math
 
 import numpy as np
@@ -54,9 +55,14 @@ class _RingGrid:
         north = [self.nlon_ring(j) for j in range(self.nlat_half)]
         return np.array(north + north[::-1])
 
-    @property
+    # kept with the grid, as every transform call compares sizes with it, until an attribute is set
+    @functools.cached_property
     def npoints(self) -> int:
-        return int(self.nlons.sum())
+        return 2 * sum(self.nlon_ring(j) for j in range(self.nlat_half))
+
+    def __setattr__(self, name, value):
+        super().__setattr__(name, value)
+        self.__dict__.pop("npoints", None)
 
     @property
     def nlon_max(self) -> int:
@@ -81,10 +87,6 @@ class OctahedralGaussianGrid(_RingGrid):
     def nlon_ring(self, j: int) -> int:
         return 16 + 4 * (j + 1)
 
-    @property
-    def npoints(self) -> int:  # the sum, in closed form: every transform call compares sizes with it
-        return 4 * self.nlat_half * (self.nlat_half + 9)
-
 
 class FullGaussianGrid(_RingGrid):
     """4 nlat_half points on every ring."""
@@ -92,10 +94,6 @@ class FullGaussianGrid(_RingGrid):
 
     def nlon_ring(self, j: int) -> int:
         return 4 * self.nlat_half
-
-    @property
-    def npoints(self) -> int:
-        return 8 * self.nlat_half * self.nlat_half
 
 
 class Field:

@@ -2,6 +2,7 @@
 (LowerTriangularArrays/src/spectrum.jl:6-70, lower_triangular_array.jl:10-20,367-395)."""
 from __future__ import annotations
 
+import functools
 import math
 
 import numpy as np
@@ -24,10 +25,15 @@ class Spectrum:
         """Spectrum(truncation; one_degree_more) (spectrum.jl:72-78)."""
         return cls(truncation + int(one_more_degree), truncation)
 
-    @property
+    # kept with the spectrum, as every transform call compares sizes with it, until an attribute is set
+    @functools.cached_property
     def nharm(self) -> int:
         """nonzeros (spectrum.jl:87-89)."""
         return self.lmax * self.mmax - self.mmax * (self.mmax - 1) // 2
+
+    def __setattr__(self, name, value):
+        super().__setattr__(name, value)
+        self.__dict__.pop("nharm", None)
 
     def offset(self, m: int) -> int:
         """0-based packed start of order m (0-based)."""
