@@ -54,6 +54,22 @@ KAPPA = R_DRY / CP
 
 
 _version, _requires_grad = operator.attrgetter("_version"), operator.attrgetter("requires_grad")
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def _plain(t, shape) -> bool:
+    """t is memory: a tensor of that shape with nothing to differentiate (nor to map through:
+    _untraced)."""
+    return type(t) in _TENSORS and t.shape == shape and not (t.requires_grad and torch.is_grad_enabled())
+
+
+def _real(t, shape) -> bool:
+    return _plain(t, shape) and not t.is_complex()
+
+
+def _untraced() -> bool:
+    """No transform of functions (vmap, jvp, ...) and no forward differentiation is on."""
+    return torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
 
 
 def _eps(l, m):
@@ -211,19 +227,8 @@ class DryPrimitiveModel:
     # last part of step), which take whatever torch takes, and as the library's kernels, 6 to 24
     # times faster (8 members and levels: T127 1.2 -> 0.19 ms per step, T31 1.1 -> 0.05), which
     # read raw memory of one form.  The kernels run where the model is as it was built
-    # (_kernels) and the tensors have that form (_plain, _columns); both give the same values.
+    # (_kernels) and the tensors have that form (_real, _columns); both give the same values.
     # A step spends its host time on these checks, so each looks at a thing once.
-    @staticmethod
-    def _plain(t, shape) -> bool:
-        """t is memory: a tensor of that shape with nothing to differentiate (nor to map
-        through: _untraced)."""
-        return (type(t) in _TENSORS and t.shape == shape and not (t.requires_grad and torch.is_grad_enabled()))
-
-    @staticmethod
-    def _untraced() -> bool:
-        """No transform of functions (vmap, jvp, ...) and no forward differentiation is on."""
-        return torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
-
     def _tables(self) -> tuple:
         return (self.sigma_half, self.sigma_full, self.G, *vars(self.ops).values())
 
@@ -231,19 +236,20 @@ class DryPrimitiveModel:
         """The library's kernels state this model: nothing that they have built in was replaced
         or written to (sigma levels, geopotential matrix, operators, transforms, methods), and
         the tables that they read hold one real value per grid point."""
-        S, grid, tables = self.S, (self.grid.npoints,), self._tables()
-        return (self._untraced()
+        S, grid, tables, E, L = self.S, (self.grid.npoints,), self._tables(), self.E, self.L
+        return (_untraced()
                 and _methods(type(self)) == _METHODS_AS_BUILT and _METHODS.isdisjoint(vars(self))
                 and type(self.ops) is SpectralOps and _operators(SpectralOps) == _OPERATORS_AS_BUILT
-                and isinstance(self.dsigma, float) and (self.L, self.dsigma) == self._levels
+                and isinstance(self.dsigma, float) and (L, self.dsigma) == self._levels
                 and len(tables) == len(self._built) and all(map(operator.is_, tables, self._built))
                 and list(map(_version, tables)) == self._writes
                 and not (torch.is_grad_enabled() and any(map(_requires_grad, tables)))
-                and type(S) is SpectralTransform and S.spectrum == self.spectrum and S.grid == self.grid
-                and S.nlayers >= self.E * max(6 * self.L + 1, 5 * self.L + 3) and S.device == self._dev.index
+                and type(S) is SpectralTransform and S.device == self._dev.index
+                and (S.spectrum is self.spectrum or S.spectrum == self.spectrum)
+                and (S.grid is self.grid or S.grid == self.grid)
+                and S.nlayers >= E * (6 * L + 1) and (L > 1 or S.nlayers >= 8 * E)
                 and isinstance(self.a, (int, float)) and self.a > 0
-                and self._plain(self.f, grid) and self._plain(self.coslat_inv, grid)
-                and not self.f.is_complex() and not self.coslat_inv.is_complex())
+                and _real(self.f, grid) and _real(self.coslat_inv, grid))
 
     def _columns(self, st: dict):
         """Device pointers of a state's vor, div, temp (E*L, nharm) and lnps (E, nharm), and the
@@ -252,7 +258,7 @@ class DryPrimitiveModel:
         keep, ptr = [], []
         for name, rows in (("vor", EL), ("div", EL), ("temp", EL), ("lnps", E)):
             t = st[name] if name in st else None
-            if not self._plain(t, (rows, n)) or t.dtype != torch.complex64 or t.device != self._dev:
+            if not _plain(t, (rows, n)) or t.dtype is not torch.complex64 or t.device != self._dev:
                 return None
             if not t.is_contiguous() or t.is_conj() or t.is_neg():
                 t = t.resolve_conj().resolve_neg().contiguous()
@@ -281,7 +287,7 @@ class DryPrimitiveModel:
         return {"vor": vor, "div": div, "temp": temp, "lnps": lnps}
 
     def _vector(self, x: torch.Tensor) -> torch.Tensor:
-        if x.dtype == torch.float32 and x.device == self._dev and x.is_contiguous() and not x.is_neg():
+        if x.dtype is torch.float32 and x.device == self._dev and x.is_contiguous() and not x.is_neg():
             return x
         return x.to(device=self._dev, dtype=torch.float32).resolve_neg().contiguous()
 
@@ -382,14 +388,16 @@ class DryPrimitiveModel:
         """_columns of the state, of the previous one and of the tendencies (None: none) where
         the time-step kernels state the step; otherwise None."""
         n, now, prev = (self.spectrum.nharm,), self.state, self.state_prev
-        if not (self._untraced() and type(self)._diffuse is _DIFFUSE and "_diffuse" not in vars(self)
+        if not (_untraced() and type(self)._diffuse is _DIFFUSE and "_diffuse" not in vars(self)
                 and isinstance(self.dt, (int, float)) and isinstance(self.robert, (int, float))
-                and isinstance(self.williams, (int, float)) and self._plain(self.nu, n) and self._plain(self.nu_div, n)
-                and not self.nu.is_complex() and not self.nu_div.is_complex() and len(now) == 4):
+                and isinstance(self.williams, (int, float)) and _real(self.nu, n) and _real(self.nu_div, n)
+                and len(now) == 4):
             return None
-        columns = [None if st is None else self._columns(st) for st in (now, prev, tend)]
-        if any(c is None and st is not None for c, st in zip(columns, (now, prev, tend))):
-            return None
+        columns = []
+        for st in (now, prev, tend):
+            columns.append(None if st is None else self._columns(st))
+            if columns[-1] is None and st is not None:
+                return None
         return columns
 
     def step(self, correction=None):
@@ -500,10 +508,9 @@ class DryPrimitiveModel:
         self.S.close()
 
 
-# The methods and operators that the kernels stand for, and the tensors that are plain memory.
+# The methods and operators that the kernels stand for.
 _TENDENCIES, _DIFFUSE = DryPrimitiveModel.tendencies, DryPrimitiveModel._diffuse
 _METHODS = {"_lta", "synth", "analyse", "uv", "_tendencies_arrays"}
 _methods = operator.attrgetter(*_METHODS)
 _operators = operator.attrgetter("dlambda", "coslat_dlat", "divergence", "curl", "laplace")
 _METHODS_AS_BUILT, _OPERATORS_AS_BUILT = _methods(DryPrimitiveModel), _operators(SpectralOps)
-_TENSORS = (torch.Tensor, torch.nn.Parameter)
