@@ -14,7 +14,7 @@
 // across the workgroup with one thread per butterfly and group of columns.
 //
 // Bound by the chain of load, passes with a barrier each, and store, at 5 or 6 workgroups per CU:
-// T255 K=64 takes 26.2 (synthesis) and 28.1 us (analysis), 15 of them what a copy of its traffic
+// T255 K=64 takes 26.2 (synthesis) and 27.1 us (analysis), 15 of them what a copy of its traffic
 // takes, about 6 each the prime and the register passes.  All global loads of a workgroup are one
 // phase, and the synthesis's last pass stores the grid (before: 30.6 and 30.0 us).
 #include "sht_device.h"
