@@ -414,7 +414,7 @@ class DryPrimitiveModel:
             tend, grid = (out if need_grid else (out, None))
             if correction is not None:
                 correction(self, tend, grid)
-            columns = self._step_kernels(tend)
+            columns = None if tend is None else self._step_kernels(tend)
         dt2 = self.dt if self.state_prev is None else 2.0 * self.dt
         w1 = self.robert * self.williams / 2
         w2 = self.robert * (1 - self.williams) / 2

@@ -154,6 +154,22 @@ def test_gradient_of_a_correction(sw, gpu):
     assert not m.state["vor"].requires_grad
 
 
+def test_missing_tendencies_raise(sw, gpu):
+    class Nothing(sw.dycore.DryPrimitiveModel):
+        def tendencies(self, st, with_grid=False):
+            pass
+    m = Nothing(21, 3)
+    m.set_state(state(sw, m, 9))
+    with pytest.raises(TypeError):
+        m.step()
+    m.close()
+
+    def drop(model, tend, grid):
+        del tend["div"]
+    with pytest.raises(KeyError):
+        steps(sw, lambda m: None, drop)
+
+
 def test_unchanged_models_run_on_the_kernels(sw, gpu):
     with torch.inference_mode():
         a = sw.dycore.DryPrimitiveModel(21, 3)
